@@ -283,7 +283,8 @@ def run_leg(args, pool: LayerPool, workload: str, headline: bool) -> dict:
     ops_gu = 2.0 * R * 2 * F * H      # the GEMMs' multiply-adds x2 (quant x quant), gate + up
     ops_dn = 2.0 * R * H * F
     layer_ops = ops_gu + ops_dn
-    mfma_path = T >= 128               # the library's default switch to the grouped f16-MFMA GEMMs
+    # the library's default switch to the f16-MFMA GEMMs: the rows that an expert averages (with copies)
+    mfma_path = T >= 128 and T * K >= (26 if spec.wtype == TYPE_Q4_0 else 30) * E
 
     log(f"warmup {warmup} steps")
     for i in range(warmup):
@@ -352,10 +353,10 @@ def run_leg(args, pool: LayerPool, workload: str, headline: bool) -> dict:
         # the combine runs in the down kernel: events [3] and [4] are back to back
         phases = {"route": phase_us[0], "gate_up": phase_us[1], "down_combine": phase_us[2] + phase_us[3]}
     else:
-        # MFMA path: SwiGLU and the Q8_0 of h run in the gate/up kernel; the exact
+        # SwiGLU and the Q8_0 of h run in the gate/up kernel; on the f16 path the exact
         # recomputation of uncertain h values precedes the down kernel
         phases = {"route": phase_us[0], "gate_up": phase_us[1],
-                  ("fixup_down" if mfma_path else "hquant_down"): phase_us[2], "combine": phase_us[3]}
+                  ("fixup_down" if mfma_path else "down"): phase_us[2], "combine": phase_us[3]}
     log("phase us: " + ", ".join(f"{k} {v:.2f}" for k, v in phases.items()))
 
     # HBM traffic per launch of the dominant kernel, measured by rocprofv3 FETCH_SIZE /
@@ -377,8 +378,9 @@ def run_leg(args, pool: LayerPool, workload: str, headline: bool) -> dict:
             gu_kernel = (f"k_gateup_q (routed gate+up expert GEMV with {'GeGLU' if geglu else 'SwiGLU'} and Q8_0 of h, "
                          "one Q8_0 block per workgroup)")
         else:
-            gu_bytes = (D_prof + S) * 2 * F * rb_h + T * (H + H // 32 * 8) + R * F * 8
-            gu_kernel = "k_gateup_stream (gate+up expert GEMV, prefetching persistent waves)"
+            gu_bytes = (D_prof + S) * 2 * F * rb_h + T * (H + H // 32 * 8) + R * (F + F // 32 * 8)
+            gu_kernel = (f"k_expert_i8<gate/up> (int8 MFMA grouped GEMM with exact f64 sums, {'GeGLU' if geglu else 'SwiGLU'} "
+                         "and Q8_0 of h in the epilogue)")
         achieved = gu_bytes / (gu_us * 1e-6) / 1e9
         roofline = {
             "bound": "hbm", "kernel": gu_kernel,

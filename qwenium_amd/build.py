@@ -21,6 +21,7 @@ SOURCES = [
     "route_kernels.hip",
     "expert_gemv_kernels.hip",
     "expert_f16_kernels.hip",
+    "expert_i8_kernels.hip",
     "misc_kernels.hip",
     "qmoe_api.cpp",
     "gguf.cpp",

@@ -847,10 +847,6 @@ static F16Args base_f16_args(const LayerDesc& L, const Workspace& ws) {
     return a;
 }
 
-static int f16_max_tiles(const LayerDesc& L, const Workspace& ws, int T) {
-    return min(ws.max_tiles, (T * L.K + kTM - 1) / kTM + min(L.E, T * L.K) + (L.S ? (T + kTM - 1) / kTM : 0));
-}
-
 template <typename Kern>
 static hipError_t launch_f16(Kern kern, dim3 grid, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop,
                              const F16Args& a) {
@@ -874,7 +870,7 @@ hipError_t launch_gateup_mfma(const LayerDesc& L, const Workspace& ws, int T, hi
     a.n_y = L.F / 64;
     // the fixup list starts empty: the routing's expert scan clears its counter
     hipError_t err = hipSuccess;
-    const dim3 grid(8 * ((f16_max_tiles(L, ws, T) + 7) / 8) * a.n_y);
+    const dim3 grid(8 * ((std::min(ws.max_tiles, max_row_tiles(L, T, kTM)) + 7) / 8) * a.n_y);
     const bool gelu = L.act == kActGeluTanh;
     if (L.gu_type == kTypeQ4_0)
         err = gelu ? launch_f16(k_expert_f16<kTypeQ4_0, true, kActGeluTanh>, grid, stream, ev_start, ev_stop, a)
@@ -909,7 +905,7 @@ hipError_t launch_down_mfma(const LayerDesc& L, const Workspace& ws, int T, hipS
     a.a_q = ws.h_q; a.a_d = ws.h_d;
     a.K = L.F;
     a.n_y = L.H / 128;
-    const dim3 grid(8 * ((f16_max_tiles(L, ws, T) + 7) / 8) * a.n_y);
+    const dim3 grid(8 * ((std::min(ws.max_tiles, max_row_tiles(L, T, kTM)) + 7) / 8) * a.n_y);
     return L.dn_type == kTypeQ4_0 ? launch_f16(k_expert_f16<kTypeQ4_0, false, kActSilu>, grid, stream, nullptr, nullptr, a)
                                   : launch_f16(k_expert_f16<kTypeQ8_0, false, kActSilu>, grid, stream, nullptr, nullptr, a);
 }

@@ -14,6 +14,7 @@
 #include "qmoe_internal.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace qmoe {
 
@@ -37,250 +38,6 @@ struct ExpertArgs {
     int sd_blocks;                             // fused decode gate/up: leading workgroups computing ysh
 };
 
-// Loads the slot table into LDS (all E+1 entries; those past n_active are
-// never read) and returns n_active.  One latency at kernel start.
-__device__ __forceinline__ int stage_slots(const ExpertArgs& a, int4* s_slots, int* s_nact) {
-    for (int i = threadIdx.x; i <= a.E; i += blockDim.x) s_slots[i] = a.slot_info[i];
-    if (threadIdx.x == 0) *s_nact = a.counters[0];
-    __syncthreads();
-    return *s_nact;
-}
-
-// ---------------------------------------------------------------------------
-// G1: gate + up projections -> gubuf (f32 pairs), persistent streaming.
-// Work item = (active slot, group of RPW consecutive ffn rows of gate and up).
-// Items are strided over all waves (consecutive waves take consecutive row
-// groups of one expert); each wave prefetches the next item's weights and
-// first-token activations while it computes the current item.  LPR lanes
-// cover one H row (lane lp owns 64-value pair lp); RPI = 64/LPR rows per load
-// instruction, NI = RPW/RPI loads per matrix.
-// ---------------------------------------------------------------------------
-template <int WT, int LPR, int RPW>
-struct GuItem {
-    static constexpr int RPI = 64 / LPR;
-    static constexpr int NI = RPW / RPI;
-    WPair<WT> wg[NI], wu[NI];
-    XPair x;
-    int e, p0, nrows, f0, t0;  // t0: the shared expert's first token (its rows are tokens t0, t0 + 1, ...)
-};
-
-// The shared expert's rows (one per token) go to items of kShChunk rows each, so
-// that no item walks all T rows one after another.
-constexpr int kShChunk = 8;
-__device__ __forceinline__ int sh_chunks(const ExpertArgs& a) { return a.S ? (a.T + kShChunk - 1) / kShChunk : 0; }
-// Slot entry of item `item` (ips items per slot or shared chunk): the shared
-// expert's chunks first (the heaviest items), then the routed experts' slots.
-__device__ __forceinline__ int4 item_slot_info(const ExpertArgs& a, const int4* slots, int item, int ips, int n_act) {
-    const int k = item / ips, nsh = sh_chunks(a);
-    if (k < nsh) {
-        const int c0 = k * kShChunk;
-        return make_int4(a.E, a.T * a.K + c0, min(kShChunk, a.T - c0), c0);
-    }
-    return slots[k - nsh];
-}
-
-// Activation source of the gate/up kernel: the quantized token rows and the
-// row -> token map, in LDS (decode: staged once per block) or in global memory.
-struct XSrc {
-    const int8_t* qs;     // [T][H]
-    const float2* ds;     // [T][H/32]
-    const int32_t* rtok;  // [R]
-};
-
-// Weights of one item (RPW rows of gate and of up of the slot's expert).
-template <int WT, int LPR, int RPW>
-__device__ __forceinline__ void gu_load_w(const ExpertArgs& a, const int4 si, int item, int ips, int sub, int lp,
-                                          GuItem<WT, LPR, RPW>& it) {
-    constexpr int RPI = 64 / LPR;
-    constexpr int NI = RPW / RPI;
-    it.e = si.x; it.p0 = si.y; it.nrows = si.z; it.t0 = si.w;
-    it.f0 = (item % ips) * RPW;
-    const bool sh = it.e >= a.E;
-    const uint8_t* gb = sh ? a.w_sh_gate : a.w_gate + (uint64_t)it.e * a.gate_nb2;
-    const uint8_t* ub = sh ? a.w_sh_up : a.w_up + (uint64_t)it.e * a.up_nb2;
-    const uint64_t gnb1 = sh ? a.sh_gate_nb1 : a.gate_nb1;
-    const uint64_t unb1 = sh ? a.sh_up_nb1 : a.up_nb1;
-    const int pair = min(lp, (a.H >> 6) - 1);  // lanes past the row re-read the last pair; their sums are dropped
-#pragma unroll
-    for (int m = 0; m < NI; ++m) {
-        const int f = it.f0 + m * RPI + sub;
-        it.wg[m].load(gb + (uint64_t)f * gnb1, pair);
-        it.wu[m].load(ub + (uint64_t)f * unb1, pair);
-    }
-}
-
-// Activations of the item's first row (token tok).
-template <int WT, int LPR, int RPW>
-__device__ __forceinline__ void gu_load_x(const ExpertArgs& a, const XSrc& xs, int tok, int lp,
-                                          GuItem<WT, LPR, RPW>& it) {
-    it.x.load(xs.qs + (uint64_t)tok * a.H, xs.ds + (uint64_t)tok * (a.H >> 5), min(lp, (a.H >> 6) - 1));
-}
-
-template <int WT, int LPR, int RPW>
-__device__ __forceinline__ void gu_load(const ExpertArgs& a, const XSrc& xs, const int4* s_slots, int n_act, int item,
-                                        int ips, int sub, int lp, GuItem<WT, LPR, RPW>& it) {
-    const int4 si = item_slot_info(a, s_slots, item, ips, n_act);
-    gu_load_w(a, si, item, ips, sub, lp, it);
-    gu_load_x(a, xs, si.w, lp, it);
-}
-
-template <int WT, int LPR, int RPW>
-__device__ __forceinline__ void gu_compute(const ExpertArgs& a, const XSrc& xs, const GuItem<WT, LPR, RPW>& it,
-                                           int sub, int lp) {
-    constexpr int RPI = 64 / LPR;
-    constexpr int NI = RPW / RPI;
-    const bool live = lp < (a.H >> 6);
-    XPair x = it.x, xn;
-    for (int c = 0; c < it.nrows; ++c) {
-        if (c + 1 < it.nrows) {  // the next row's activations, requested before this row's dots
-            const int tok = it.e >= a.E ? it.t0 + c + 1 : xs.rtok[it.p0 + c + 1];
-            xn.load(xs.qs + (uint64_t)tok * a.H, xs.ds + (uint64_t)tok * (a.H >> 5), min(lp, (a.H >> 6) - 1));
-        }
-#pragma unroll
-        for (int m = 0; m < NI; ++m) {
-            double g, u;
-            group_sum2_f64<LPR>(live ? pair_dot<WT>(it.wg[m], x) : 0.0, live ? pair_dot<WT>(it.wu[m], x) : 0.0, g, u);
-            float2& o = a.gubuf[(uint64_t)(it.p0 + c) * a.F + it.f0 + m * RPI + sub];
-            if constexpr (LPR >= 32) {
-                if (lp == LPR / 2 - 1) o.x = (float)g;
-                if (lp == LPR - 1) o.y = (float)u;
-            } else {
-                if (lp == LPR - 1) o = make_float2((float)g, (float)u);
-            }
-        }
-        x = xn;
-    }
-}
-
-// Token rows staged in LDS by the gate/up kernel: at most 32 KiB of quants
-// (8 chunks of 16 bytes per thread of a 256-thread block).
-constexpr int kGuStageChunks = 8;
-
-// LDS layout of the gate/up kernel: slot table, then (XLDS) the T quantized
-// token rows, their scales and the row -> token map.
-__host__ __device__ constexpr size_t gu_lds_slots(int E) { return (size_t)(E + 1) * 16; }
-__host__ __device__ constexpr size_t gu_lds_bytes(int E, int T, int H, int R, bool xlds) {
-    return gu_lds_slots(E) + (xlds ? (size_t)T * H + (size_t)T * (H / 32) * 8 + (size_t)((R + 3) & ~3) * 4 : 0);
-}
-
-// Copies n (>= 1) 16-byte chunks global -> LDS with all of a thread's loads
-// (at most MAXC) issued before its first store: one memory round trip.  Loads
-// past n re-read the last chunk (unconditional loads keep v[] in registers).
-template <int MAXC>
-__device__ __forceinline__ void stage_chunks(u32x4* dst, const u32x4* src, int n) {
-    u32x4 v[MAXC];
-#pragma unroll
-    for (int u = 0; u < MAXC; ++u) v[u] = src[min((int)threadIdx.x + 256 * u, n - 1)];
-#pragma unroll
-    for (int u = 0; u < MAXC; ++u) {
-        const int i = threadIdx.x + 256 * u;
-        if (i < n) dst[i] = v[u];
-    }
-}
-
-template <int WT, int LPR, int RPW, bool XLDS>
-__global__ __launch_bounds__(256) void k_gateup_stream(ExpertArgs a) {
-    extern __shared__ __align__(16) uint8_t s_dyn[];
-    int4* s_slots = (int4*)s_dyn;
-    // routed slots (the table's last slot is the shared expert's, which goes to chunks)
-    const int n_act = __builtin_amdgcn_readfirstlane(a.counters[0]) - a.S;
-    const int ips = a.F / RPW;
-    const int n_items = (n_act + sh_chunks(a)) * ips;
-    const int lane = threadIdx.x & 63;
-    const int sub = lane / LPR, lp = lane % LPR;
-    const int tw = gridDim.x * (blockDim.x >> 6);
-    int item = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // ping-pong: while one buffer is computed the other one's loads are in flight.  The
-    // first two items' weights are requested before the block stages its tables, with
-    // their slot entries read from global memory.
-    GuItem<WT, LPR, RPW> b0, b1;
-    int4 si0 = make_int4(0, 0, 0, 0), si1 = si0;
-    if (item < n_items) {
-        si0 = item_slot_info(a, a.slot_info, item, ips, n_act);
-        gu_load_w(a, si0, item, ips, sub, lp, b0);
-        if (item + tw < n_items) {
-            si1 = item_slot_info(a, a.slot_info, item + tw, ips, n_act);
-            gu_load_w(a, si1, item + tw, ips, sub, lp, b1);
-        }
-    }
-    XSrc xs{a.xq_qs, a.xq_ds, a.row_token};
-    if (XLDS) {
-        // the T token rows (16-byte chunks), their scales and the row map
-        int8_t* lq = (int8_t*)(s_dyn + gu_lds_slots(a.E));
-        float2* ld = (float2*)(lq + (size_t)a.T * a.H);
-        int32_t* lr = (int32_t*)(ld + (size_t)a.T * (a.H >> 5));
-        const int nq = a.T * a.H / 16, nd = a.T * (a.H >> 5) / 2, R = a.offsets[a.E + 1];
-        stage_chunks<kGuStageChunks>((u32x4*)lq, (const u32x4*)a.xq_qs, nq);
-        stage_chunks<2>((u32x4*)ld, (const u32x4*)a.xq_ds, nd);
-        for (int i = threadIdx.x; i < R; i += blockDim.x) lr[i] = a.row_token[i];
-        xs = XSrc{lq, ld, lr};
-    }
-    for (int i = threadIdx.x; i < n_act; i += blockDim.x) s_slots[i] = a.slot_info[i];
-    __syncthreads();
-    if (item >= n_items) return;
-    gu_load_x(a, xs, si0.w, lp, b0);
-    if (item + tw < n_items) gu_load_x(a, xs, si1.w, lp, b1);
-    for (;;) {
-        int nitem = item + tw;
-        gu_compute(a, xs, b0, sub, lp);
-        if (nitem >= n_items) break;
-        item = nitem;
-        nitem = item + tw;
-        if (nitem < n_items) gu_load(a, xs, s_slots, n_act, nitem, ips, sub, lp, b0);
-        gu_compute(a, xs, b1, sub, lp);
-        if (nitem >= n_items) break;
-        item = nitem;
-        nitem = item + tw;
-        if (nitem < n_items) gu_load(a, xs, s_slots, n_act, nitem, ips, sub, lp, b1);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Q: h = silu(g)*u (SwiGLU) or gelu(g)*u (GeGLU) of each (row, ffn index), then Q8_0 quantization of
-// the h rows (the activation quantization ggml applies to src1 of the down
-// mul_mat_id).  Each lane takes 4 consecutive values; the 8 lanes of a 32-value
-// block reduce with DPP (quad xor 1, quad xor 2, half-row mirror) and store
-// their quants as one dword each.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_quant_h(ExpertArgs a) {
-    const int nrows = a.offsets[a.E + 1];
-    const int nq = a.F >> 2;  // quads per row (a multiple of 16: blocks never straddle rows or waves)
-    const int gq = blockIdx.x * 256 + threadIdx.x;
-    if ((gq & ~63) >= nrows * nq) return;  // whole waves past the end
-    const bool live = gq < nrows * nq;     // uniform over each 8-lane block
-    const int gqc = live ? gq : 0;
-    const int p = gqc / nq, q = gqc - p * nq;
-    const f32x4* src = (const f32x4*)(a.gubuf + (uint64_t)p * a.F + 4 * q);
-    const f32x4 v0 = src[0], v1 = src[1];  // (g0, u0, g1, u1), (g2, u2, g3, u3)
-    float h[4];
-    h[0] = act_mul(a.act, a.gelu_tab, v0.x, v0.y);
-    h[1] = act_mul(a.act, a.gelu_tab, v0.z, v0.w);
-    h[2] = act_mul(a.act, a.gelu_tab, v1.x, v1.y);
-    h[3] = act_mul(a.act, a.gelu_tab, v1.z, v1.w);
-    float amax = fmaxf(fmaxf(__builtin_fabsf(h[0]), __builtin_fabsf(h[1])),
-                       fmaxf(__builtin_fabsf(h[2]), __builtin_fabsf(h[3])));
-    amax = dpp8_max<kDppQuadXor1>(amax);
-    amax = dpp8_max<kDppQuadXor2>(amax);
-    amax = dpp8_max<kDppRowHalfMirror>(amax);
-    const float d = amax / 127.0f;
-    const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
-    uint32_t word = 0;
-    int sum = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int qv = (int)__builtin_rintf(h[i] * id);
-        sum += qv;
-        word |= ((uint32_t)qv & 0xffu) << (8 * i);
-    }
-    sum = dpp8_add<kDppQuadXor1>(sum);
-    sum = dpp8_add<kDppQuadXor2>(sum);
-    sum = dpp8_add<kDppRowHalfMirror>(sum);
-    if (!live) return;
-    *(uint32_t*)(a.hq_qs + (uint64_t)p * a.F + 4 * q) = word;
-    if ((q & 7) == 0)
-        a.hq_ds[(uint64_t)p * (a.F >> 5) + (q >> 3)] = make_float2(fp16_to_f32(f32_to_fp16(d)), __builtin_bit_cast(float, sum));
-}
-
 // ---------------------------------------------------------------------------
 // G1+Q at decode sizes: gate/up, SwiGLU and the Q8_0 quantization of h of the
 // routed experts in one launch (the decode routing launch does the shared
@@ -289,7 +46,8 @@ __global__ __launch_bounds__(256) void k_quant_h(ExpertArgs a) {
 // The block stages its slot's token rows (Q8_0 of x) in LDS -- loads issued
 // before the weight loads, so they land first -- computes g and u for every
 // row into LDS, then one lane per value does h = silu(g)*u and 32 lanes
-// quantize a row's block: the same operations as k_quant_h, so the same bits.
+// quantize a row's block: the
+// operations of swiglu_q8_block32, as in every path, so the same bits.
 // ---------------------------------------------------------------------------
 
 #ifndef GQ_Q4_WAVES
@@ -488,111 +246,6 @@ __global__ __launch_bounds__(NW * 64, GQ_MIN_WAVES) void k_gateup_q(ExpertArgs a
         const int p = p0 + c;
         swiglu_q8_block32(gu.x, gu.y, fl, a.hq_qs + (uint64_t)p * a.F + fb * 32, a.hq_ds + (uint64_t)p * nfb + fb,
                           a.act, a.gelu_tab);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// G2: down projection, persistent streaming.  Work item = (active slot, group
-// of RPW consecutive output rows n).  LPR lanes per F row.  Writes ybuf[p][n].
-// ---------------------------------------------------------------------------
-template <int WT, int LPR, int RPW>
-struct DnItem {
-    static constexpr int RPI = 64 / LPR;
-    static constexpr int NI = RPW / RPI;
-    WPair<WT> w[NI];
-    XPair x;
-    int e, p0, nrows, n0, t0;  // t0: the shared expert's first token
-};
-
-template <int WT, int LPR, int RPW>
-__device__ __forceinline__ void dn_load(const ExpertArgs& a, const XSrc& hs, const int4* s_slots, int item, int ips,
-                                        int sub, int lp, int n_act, DnItem<WT, LPR, RPW>& it) {
-    constexpr int RPI = 64 / LPR;
-    constexpr int NI = RPW / RPI;
-    const int4 si = item_slot_info(a, s_slots, item, ips, n_act);
-    it.e = si.x; it.p0 = si.y; it.nrows = si.z; it.t0 = si.w;
-    it.n0 = (item % ips) * RPW;
-    const bool sh = it.e >= a.E;
-    const uint8_t* db = sh ? a.w_sh_down : a.w_down + (uint64_t)it.e * a.down_nb2;
-    const uint64_t dnb1 = sh ? a.sh_down_nb1 : a.down_nb1;
-    const int pair = min(lp, (a.F >> 6) - 1);
-#pragma unroll
-    for (int m = 0; m < NI; ++m) it.w[m].load(db + (uint64_t)(it.n0 + m * RPI + sub) * dnb1, pair);
-    if (sh && hs.qs) it.x.load(hs.qs + (uint64_t)it.t0 * a.F, hs.ds + (uint64_t)it.t0 * (a.F >> 5), pair);  // uniform branches keep the address spaces known
-    else it.x.load(a.hq_qs + (uint64_t)it.p0 * a.F, a.hq_ds + (uint64_t)it.p0 * (a.F >> 5), pair);
-}
-
-template <int WT, int LPR, int RPW>
-__device__ __forceinline__ void dn_compute(const ExpertArgs& a, const XSrc& hs, const DnItem<WT, LPR, RPW>& it,
-                                           int sub, int lp) {
-    constexpr int RPI = 64 / LPR;
-    constexpr int NI = RPW / RPI;
-    const bool live = lp < (a.F >> 6);
-    const bool sh = it.e >= a.E;
-    XPair x = it.x, xn;
-    for (int c = 0; c < it.nrows; ++c) {
-        const int p = it.p0 + c;
-        if (c + 1 < it.nrows) {
-            // the next row, requested before this row's dots: shared-expert rows from
-            // the block's LDS copy (hs), routed rows from global memory
-            const int pair = min(lp, (a.F >> 6) - 1);
-            const int tn = it.t0 + c + 1;
-            if (sh && hs.qs) xn.load(hs.qs + (uint64_t)tn * a.F, hs.ds + (uint64_t)tn * (a.F >> 5), pair);
-            else xn.load(a.hq_qs + (uint64_t)(p + 1) * a.F, a.hq_ds + (uint64_t)(p + 1) * (a.F >> 5), pair);
-        }
-#pragma unroll
-        for (int m = 0; m < NI; ++m) {
-            const double y = dpp_sum_f64<LPR>(live ? pair_dot<WT>(it.w[m], x) : 0.0);
-            if (lp == LPR - 1) a.ybuf[(uint64_t)p * a.H + it.n0 + m * RPI + sub] = (float)y;
-        }
-        x = xn;
-    }
-}
-
-// LDS of the down kernel: slot table, then (SHLDS) the shared expert's T rows
-// of quantized h (the slot with the most rows at decode sizes).
-__host__ __device__ constexpr size_t dn_lds_bytes(int E, int T, int F, bool shlds) {
-    return (size_t)(E + 1) * 16 + (shlds ? (size_t)T * F + (size_t)T * (F / 32) * 8 : 0);
-}
-
-template <int WT, int LPR, int RPW, bool SHLDS>
-__global__ __launch_bounds__(256) void k_down_stream(ExpertArgs a) {
-    extern __shared__ __align__(16) uint8_t s_dyn[];
-    __shared__ int s_nact;
-    int4* s_slots = (int4*)s_dyn;
-    XSrc hs{nullptr, nullptr, nullptr};
-    if (SHLDS) {
-        int8_t* lq = (int8_t*)(s_dyn + (size_t)(a.E + 1) * 16);
-        float2* ld = (float2*)(lq + (size_t)a.T * a.F);
-        const int A = a.T * a.K;  // the shared rows follow the T*K routed rows
-        const int nq = a.T * a.F / 16, nd = a.T * (a.F >> 5) / 2;
-        const u32x4* gq = (const u32x4*)(a.hq_qs + (uint64_t)A * a.F);
-        const u32x4* gd = (const u32x4*)(a.hq_ds + (uint64_t)A * (a.F >> 5));
-        for (int i = threadIdx.x; i < nq; i += blockDim.x) ((u32x4*)lq)[i] = gq[i];
-        for (int i = threadIdx.x; i < nd; i += blockDim.x) ((u32x4*)ld)[i] = gd[i];
-        hs = XSrc{lq, ld, nullptr};
-    }
-    const int n_act = stage_slots(a, s_slots, &s_nact) - a.S;  // routed slots; the shared expert goes to chunks
-    const int ips = a.H / RPW;
-    const int n_items = (n_act + sh_chunks(a)) * ips;
-    const int lane = threadIdx.x & 63;
-    const int sub = lane / LPR, lp = lane % LPR;
-    const int tw = gridDim.x * (blockDim.x >> 6);
-    int item = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (item >= n_items) return;
-    DnItem<WT, LPR, RPW> b0, b1;
-    dn_load(a, hs, s_slots, item, ips, sub, lp, n_act, b0);
-    for (;;) {
-        int nitem = item + tw;
-        if (nitem < n_items) dn_load(a, hs, s_slots, nitem, ips, sub, lp, n_act, b1);
-        dn_compute(a, hs, b0, sub, lp);
-        if (nitem >= n_items) break;
-        item = nitem;
-        nitem = item + tw;
-        if (nitem < n_items) dn_load(a, hs, s_slots, nitem, ips, sub, lp, n_act, b0);
-        dn_compute(a, hs, b1, sub, lp);
-        if (nitem >= n_items) break;
-        item = nitem;
     }
 }
 
@@ -822,13 +475,27 @@ bool down_combine_tok_fits(const LayerDesc& L) {
     return nj <= 9 && dc_lds_bytes(L.F, nj) <= 64 * 1024 && dc_stage_chunks(L.F, nj) <= 1024 && L.dc_ahead <= 2;
 }
 
-// Up to 16 tokens either down+combine kernel; beyond, below the MFMA path, the
-// token-per-workgroup one (its step tables are per token; measured faster than
-// the streaming down + k_combine from 24 to 127 tokens: 99 -> 86 us at 24 tokens,
-// 156 -> 146 at 64, 221 -> 215 at 127).
+// Whether reading each token's experts' down rows for it alone (the token-per-
+// workgroup kernel, ~8.7 TB/s out of the caches) beats reading each expert's once
+// (the grouped GEMM at ~4.5 TB/s and its combine's ~8 us).  Layer us, token /
+// grouped: 35B-A3B Q4_0 93.4 / 99.4 at 32 tokens, 123.0 / 123.3 at 64, 147.7 /
+// 140.8 at 96; Q8_0 196.7 / 194.6 at 64; Gemma 4 109.7 / 116.6 at 24, 142.6 /
+// 135.8 at 48; hidden 4096, 32 experts, top-4 78.4 / 77.4 at 17, 114.0 / 88.5 at
+// 48.  From four rows per expert and 40 tokens always grouped, small layers too
+// (hidden 1024, 16 experts, top-2 35.7 / 36.6 at 32, 40.9 / 38.1 at 48).
+static bool down_per_token(const LayerDesc& L, int T) {
+    if (T >= 40 && (int64_t)T * L.K >= 4 * (int64_t)L.E) return false;
+    const int bb = L.dn_type == kTypeQ4_0 ? BlockTraits<kTypeQ4_0>::kBytes : BlockTraits<kTypeQ8_0>::kBytes;
+    const double mb = 1e-6 * L.H * (L.F / 32) * bb;  // one expert's down rows
+    const double distinct = L.E * (1.0 - std::pow(1.0 - (double)L.K / L.E, T)) + L.S;
+    return T * (L.K + L.S) * mb / 8.7 < 8.0 + distinct * mb / 4.5;
+}
+
+// Up to 16 tokens either down+combine kernel; beyond, below the f16 path, the
+// token-per-workgroup one while it is the faster (its step tables are per token).
 bool down_combine_fused(const LayerDesc& L, int T) {
-    return T < L.mfma_min_tokens && L.K + L.S <= kDcMaxSteps &&
-           (T <= kTopkTokensPerBlock || down_combine_tok_fits(L));
+    return T < mfma_from(L) && L.K + L.S <= kDcMaxSteps &&
+           (T <= kTopkTokensPerBlock || (down_combine_tok_fits(L) && down_per_token(L, T)));
 }
 
 // Up to 9 steps (8 routed + shared) whose activation rows fit in 64 KiB of
@@ -884,73 +551,6 @@ hipError_t launch_down_combine(const LayerDesc& L, const Workspace& ws, int T, f
                                     : launch_down_combine_t<kTypeQ8_0>(a, L.dc_ahead, stream);
 }
 
-// Persistent grid: every block resident at once (blocks per CU from the
-// occupancy calculator), never more waves than items.
-template <typename KernelT>
-static int stream_blocks(KernelT kernel, size_t lds, int n_items_max, int n_cu) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, lds) != hipSuccess || per_cu < 1) per_cu = 1;
-    const int want = (n_items_max + 3) / 4;
-    return std::max(1, std::min(want, n_cu * per_cu));
-}
-
-// Token rows are staged in LDS when they take at most this many bytes per block.
-constexpr size_t kGuXLdsMax = 32 * 1024;
-
-template <int WT, int LPR, int RPW>
-static hipError_t launch_gateup_v(const ExpertArgs& a, int max_slots, int n_cu, hipStream_t stream, hipEvent_t e0,
-                                  hipEvent_t e1) {
-    const int R = a.T * a.K + a.S * a.T;
-    const bool xlds = gu_lds_bytes(a.E, a.T, a.H, R, true) - gu_lds_slots(a.E) <= kGuXLdsMax;
-    const size_t lds = gu_lds_bytes(a.E, a.T, a.H, R, xlds);
-    if (xlds) {
-        auto kern = k_gateup_stream<WT, LPR, RPW, true>;
-        const int g = stream_blocks(kern, lds, max_slots * (a.F / RPW), n_cu);
-        launch_timed(kern, dim3(g), dim3(256), lds, stream, e0, e1, a);
-    } else {
-        auto kern = k_gateup_stream<WT, LPR, RPW, false>;
-        const int g = stream_blocks(kern, lds, max_slots * (a.F / RPW), n_cu);
-        launch_timed(kern, dim3(g), dim3(256), lds, stream, e0, e1, a);
-    }
-    return hipGetLastError();
-}
-
-template <int WT>
-static hipError_t launch_gateup(const ExpertArgs& a, int max_slots, int n_cu, hipStream_t stream, hipEvent_t e0,
-                                hipEvent_t e1) {
-    const int npairs = a.H / 64;
-    if (npairs <= 16) return launch_gateup_v<WT, 16, 4>(a, max_slots, n_cu, stream, e0, e1);
-    if (npairs <= 32) return launch_gateup_v<WT, 32, 4>(a, max_slots, n_cu, stream, e0, e1);  // 4 rows: twice the bytes per request (2 rows: +14%, 8 rows: +19% at 64 tokens)
-    return launch_gateup_v<WT, 64, 2>(a, max_slots, n_cu, stream, e0, e1);
-}
-
-template <int WT, int LPR>
-static hipError_t launch_down_v(const ExpertArgs& a, int max_slots, int n_cu, hipStream_t stream) {
-    constexpr int RPW = 4 * (64 / LPR);  // four load instructions per item (at 64 tokens: two +8%, one +40%, eight +25%)
-    const bool shlds = a.S && dn_lds_bytes(a.E, a.T, a.F, true) - dn_lds_bytes(a.E, a.T, a.F, false) <= kGuXLdsMax;
-    const size_t lds = dn_lds_bytes(a.E, a.T, a.F, shlds);
-    if (shlds) {
-        auto kern = k_down_stream<WT, LPR, RPW, true>;
-        const int g = stream_blocks(kern, lds, max_slots * (a.H / RPW), n_cu);
-        hipLaunchKernelGGL(kern, dim3(g), dim3(256), lds, stream, a);
-    } else {
-        auto kern = k_down_stream<WT, LPR, RPW, false>;
-        const int g = stream_blocks(kern, lds, max_slots * (a.H / RPW), n_cu);
-        hipLaunchKernelGGL(kern, dim3(g), dim3(256), lds, stream, a);
-    }
-    return hipGetLastError();
-}
-
-template <int WT>
-static hipError_t launch_down(const ExpertArgs& a, int max_slots, int n_cu, hipStream_t stream) {
-    const int npairs = a.F / 64;
-    if (npairs <= 4) return launch_down_v<WT, 4>(a, max_slots, n_cu, stream);
-    if (npairs <= 8) return launch_down_v<WT, 8>(a, max_slots, n_cu, stream);
-    if (npairs <= 16) return launch_down_v<WT, 16>(a, max_slots, n_cu, stream);
-    if (npairs <= 32) return launch_down_v<WT, 32>(a, max_slots, n_cu, stream);
-    return launch_down_v<WT, 64>(a, max_slots, n_cu, stream);
-}
-
 static ExpertArgs make_expert_args(const LayerDesc& L, const Workspace& ws, int T) {
     ExpertArgs a;
     a.H = L.H; a.F = L.F; a.E = L.E; a.K = L.K; a.S = L.S; a.T = T;
@@ -967,14 +567,6 @@ static ExpertArgs make_expert_args(const LayerDesc& L, const Workspace& ws, int 
     a.ysh = ws.ysh;
     a.sd_blocks = 0;
     return a;
-}
-
-hipError_t launch_experts_gateup(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream,
-                                 hipEvent_t ev_start, hipEvent_t ev_stop) {
-    const ExpertArgs a = make_expert_args(L, ws, T);
-    const int max_slots = min(L.E, T * L.K) + L.S;
-    return (L.gu_type == kTypeQ4_0) ? launch_gateup<kTypeQ4_0>(a, max_slots, L.n_cu, stream, ev_start, ev_stop)
-                                    : launch_gateup<kTypeQ8_0>(a, max_slots, L.n_cu, stream, ev_start, ev_stop);
 }
 
 // The fused decode gate/up needs the decode slot list (the decode routing),
@@ -1010,21 +602,6 @@ hipError_t launch_gateup_q(const LayerDesc& L, const Workspace& ws, int T, hipSt
     }
     return (L.gu_type == kTypeQ4_0) ? launch_gateup_q_t<kTypeQ4_0>(a, ws.dslots, max_v, stream, ev_start, ev_stop)
                                     : launch_gateup_q_t<kTypeQ8_0>(a, ws.dslots, max_v, stream, ev_start, ev_stop);
-}
-
-hipError_t launch_quant_h(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream) {
-    const ExpertArgs a = make_expert_args(L, ws, T);
-    const int max_rows = T * L.K + L.S * T;
-    const int qblocks = (max_rows * (L.F / 4) + 255) / 256;
-    hipLaunchKernelGGL(k_quant_h, dim3(qblocks), dim3(256), 0, stream, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_experts_down(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream) {
-    const ExpertArgs a = make_expert_args(L, ws, T);
-    const int max_slots = min(L.E, T * L.K) + L.S;
-    return (L.dn_type == kTypeQ4_0) ? launch_down<kTypeQ4_0>(a, max_slots, L.n_cu, stream)
-                                    : launch_down<kTypeQ8_0>(a, max_slots, L.n_cu, stream);
 }
 
 // ---------------------------------------------------------------------------

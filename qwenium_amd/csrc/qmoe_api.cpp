@@ -358,13 +358,22 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
     int n_cu = 0;
     if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, L->device) == hipSuccess && n_cu > 0)
         d.n_cu = n_cu;
-    // token count from which the grouped f16-MFMA GEMMs replace the streaming GEMVs:
-    // where an expert averages about 5.5 rows (T * top_k / n_experts), and from 128
-    // tokens at least (measured: the 35B-A3B shape crosses over near 176 tokens,
-    // Gemma 4's below 128)
+    // token count from which the grouped f16-MFMA GEMMs (f32 sums, 128-row tiles)
+    // replace the exact int8 ones: by the rows that an expert averages (T * top_k /
+    // n_experts), 40 (Q4_0) or 56 (Q8_0) over the GGUF rows, 26 or 30 with the
+    // chunk-major copies.  Layer us, int8 / f16: 35B-A3B Q4_0 328 / 375 at 31 rows,
+    // 423 / 408 at 44, with copies 256 / 292 at 22 and 328 / 311 at 31; Q8_0 490 /
+    // 554 at 44, 606 / 590 at 62, with copies 305 / 360 at 22 and 384 / 377 at 31;
+    // Gemma 4 292 / 343 at 28, 397 / 392 at 44, with copies 240 / 273 at 19 and 292
+    // / 284 at 28.
     {
-        const int64_t t = (11 * (int64_t)d.E + 2 * d.K - 1) / (2 * d.K);  // ceil(5.5 E / K)
-        d.mfma_min_tokens = (int)std::max<int64_t>(128, std::min<int64_t>(4096, (t + 15) / 16 * 16));
+        const bool q4 = d.gu_type == QMOE_TYPE_Q4_0;
+        auto from = [&](int rows) {
+            const int64_t t = ((int64_t)rows * d.E + d.K - 1) / d.K;
+            return (int)std::max<int64_t>(128, std::min<int64_t>(1 << 20, (t + 15) / 16 * 16));
+        };
+        d.mfma_min_tokens = from(q4 ? 40 : 56);
+        d.mfma_min_tokens_pk = from(q4 ? 26 : 30);
     }
     // token count from which routing runs the batched bf16-MFMA router: its cost is
     // nearly flat in T (its tiles split over more workgroups at small T), the exact
@@ -377,7 +386,7 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
     }
     if (const char* env = std::getenv("QMOE_MFMA_MIN_TOKENS")) {
         const long v = std::strtol(env, nullptr, 10);
-        if (v >= 1) d.mfma_min_tokens = (int)std::min<long>(v, 1 << 30);
+        if (v >= 1) d.mfma_min_tokens = d.mfma_min_tokens_pk = (int)std::min<long>(v, 1 << 30);
     }
     // decode down+combine prefetch depth (tuning)
     if (const char* env = std::getenv("QMOE_DC_AHEAD")) {
@@ -691,7 +700,7 @@ static int forward_impl(qmoe_layer* layer, qmoe_workspace* ws, const ForwardIn& 
     // the prefill GEMMs address their A operands (x and h quants as f16) with
     // 32-bit byte offsets
     const uint64_t R = (uint64_t)n_tokens * (d.K + d.S);
-    const bool mfma = n_tokens >= d.mfma_min_tokens && !qmoe::gateup_q_fused(d, n_tokens) &&
+    const bool mfma = n_tokens >= qmoe::mfma_from(d) && !qmoe::gateup_q_fused(d, n_tokens) &&
                       R * d.F * 2 + 256 < (1ull << 32) && (uint64_t)n_tokens * d.H * 2 + 256 < (1ull << 32);
     // decode: the routing normalizes x on the fly (no RMSNorm launch, no normalized copy)
     const float* route_norm_w = nullptr;
@@ -700,7 +709,7 @@ static int forward_impl(qmoe_layer* layer, qmoe_workspace* ws, const ForwardIn& 
         residual = x;
         if (!mfma && qmoe::route_norm_fused(d, n_tokens)) {
             route_norm_w = in.norm_w;
-        } else if (mfma && qmoe::route_uses_mfma(d, n_tokens) && !dbg && d.H <= 4096) {
+        } else if (qmoe::route_uses_mfma(d, n_tokens) && !dbg && d.H <= 4096) {
             // prefill: the batched router's preparation normalizes the rows (the
             // scale from x_ssq when carried) into every operand it writes, the
             // exact refinement normalizes on the fly: no normalized copy of x
@@ -718,7 +727,8 @@ static int forward_impl(qmoe_layer* layer, qmoe_workspace* ws, const ForwardIn& 
         xr = v.xr;
     }
     if (err == hipSuccess)
-        err = qmoe::launch_route(d, v, xin, xr, n_tokens, rdbg, mfma, stream, route_norm_w, in.eps, in.x_ssq);
+        err = qmoe::launch_route(d, v, xin, xr, n_tokens, rdbg, mfma,
+                                 mfma ? qmoe::kMfmaTileM : qmoe::i8_tile_rows(d, n_tokens), stream, route_norm_w, in.eps, in.x_ssq);
     if (err != hipSuccess) return hip_fail(err, "route kernels");
     // events [1] and [2] are taken by the gate/up launch itself (its own start and end)
     hipEvent_t e1 = layer->record_phases ? layer->phase_events[1] : nullptr;
@@ -732,9 +742,9 @@ static int forward_impl(qmoe_layer* layer, qmoe_workspace* ws, const ForwardIn& 
         err = qmoe::launch_gateup_mfma(d, v, n_tokens, stream, e1, e2);
         if (err != hipSuccess) return hip_fail(err, "gate/up expert kernel");
     } else {
-        err = qmoe::launch_experts_gateup(d, v, n_tokens, stream, e1, e2);
+        // few rows per expert: exact sums, SwiGLU and the Q8_0 of h in the gate/up epilogue
+        err = qmoe::launch_gateup_i8(d, v, n_tokens, stream, e1, e2);
         if (err != hipSuccess) return hip_fail(err, "gate/up expert kernel");
-        err = qmoe::launch_quant_h(d, v, n_tokens, stream);
     }
     bool ssq_done = false;
     if (qmoe::down_combine_fused(d, n_tokens)) {
@@ -744,7 +754,7 @@ static int forward_impl(qmoe_layer* layer, qmoe_workspace* ws, const ForwardIn& 
         err = mark(3);
     } else {
         if (err == hipSuccess)
-            err = mfma ? qmoe::launch_down_mfma(d, v, n_tokens, stream) : qmoe::launch_experts_down(d, v, n_tokens, stream);
+            err = mfma ? qmoe::launch_down_mfma(d, v, n_tokens, stream) : qmoe::launch_down_i8(d, v, n_tokens, stream);
         if (err != hipSuccess) return hip_fail(err, "down expert kernel");
         err = mark(3);
         if (err == hipSuccess) err = qmoe::launch_combine(d, v, n_tokens, y, residual, stream, in.y_ssq);

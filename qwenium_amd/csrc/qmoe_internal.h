@@ -53,7 +53,8 @@ struct LayerDesc {
     uint64_t sh_gate_nb1 = 0, sh_up_nb1 = 0, sh_down_nb1 = 0;
     const float* w_sh_norm = nullptr;
     int n_cu = 256;                         // compute units of the layer's device
-    int mfma_min_tokens = 128;              // token count from which the f16-MFMA GEMMs run (set per shape)
+    int mfma_min_tokens = 128;              // token count from which the f16-MFMA GEMMs run over the GGUF rows
+    int mfma_min_tokens_pk = 128;           // ... and with chunk-major copies (both set per shape)
     int big_router_min_tokens = 256;        // token count from which the bf16-MFMA router runs (set per shape)
     int dc_ahead = 2;                       // decode down+combine: steps with loads in flight (2 or 4)
     unsigned long long* expert_counts = nullptr;  // optional device [E]: += each forward's per-expert dispatches
@@ -71,6 +72,7 @@ struct LayerDesc {
     const uint8_t* pk_sh_down = nullptr;
     void* pk_base = nullptr;
 };
+inline int mfma_from(const LayerDesc& L) { return L.pk_base ? L.mfma_min_tokens_pk : L.mfma_min_tokens; }
 // The chunk-major copies (LayerDesc::pk_*) of a layer's expert matrices.
 hipError_t build_prefill_copies(LayerDesc& d);
 
@@ -126,6 +128,13 @@ struct Workspace {
     int max_tiles = 0;
 };
 
+// The most tiles of `rows` rows that a forward of T tokens lists: n rows of an expert
+// are 1 + (n - 1) / rows tiles.
+inline int max_row_tiles(const LayerDesc& L, int T, int rows) {
+    const int A = T * L.K, active = A < L.E ? A : L.E;
+    return active + (A - active) / rows + (L.S ? (T + rows - 1) / rows : 0);
+}
+
 size_t workspace_bytes(int T, int H, int E, int K, int F, Workspace* carve, void* base, bool pad = false);
 
 // Launch with optional start/stop events recorded by the launch itself.
@@ -157,6 +166,8 @@ bool route_uses_mfma(const LayerDesc& L, int T);
 bool route_decode_fused(const LayerDesc& L, int T);
 // x: the experts' input (quantized to Q8_0); xr: the router's input (x for
 // the Qwen layer; the scaled norm for Gemma 4); the shared gate reads xr.
+// tile_rows: rows per entry of the tile list, kMfmaTileM (ws.tiles) or i8_tile_rows
+// (i8_tiles, the shared expert's first).
 // x_f16: also write x's Q8_0 quants as f16 and its fp16 block scales (ws.x_q,
 // ws.x_d), the prefill GEMMs' A operand (inside the batched router's launch,
 // else a launch of its own).
@@ -165,30 +176,33 @@ bool route_decode_fused(const LayerDesc& L, int T);
 // decode (T <= 16 without x_f16, route_norm_fused says when) and in the batched
 // router (route_uses_mfma, with x_f16); x_ssq (optional): x's partial sums.
 hipError_t launch_route(const LayerDesc& L, const Workspace& ws, const float* x, const float* xr, int T,
-                        const RouteDebug& dbg, bool x_f16, hipStream_t stream, const float* norm_w = nullptr,
-                        float eps = 0.0f, const double* x_ssq = nullptr);
+                        const RouteDebug& dbg, bool x_f16, int tile_rows, hipStream_t stream,
+                        const float* norm_w = nullptr, float eps = 0.0f, const double* x_ssq = nullptr);
 bool route_norm_fused(const LayerDesc& L, int T);
 // ev_start / ev_stop (optional): events recorded at the kernel's own start and
 // end (profiling of the dominant kernel without marker overhead).
-hipError_t launch_experts_gateup(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream,
-                                 hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
-hipError_t launch_experts_down(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream);
-hipError_t launch_quant_h(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream);
 // Decode: gate/up + SwiGLU + Q8_0 of h of the routed experts in one launch
-// over ws.dslots (replaces launch_experts_gateup + launch_quant_h when
-// gateup_q_fused(); the decode routing launch computes the shared expert's h).
+// over ws.dslots (when gateup_q_fused(); the decode routing launch computes the shared expert's h).
 bool gateup_q_fused(const LayerDesc& L, int T);
 hipError_t launch_gateup_q(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream,
                            hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
 hipError_t launch_gateup_mfma(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream,
                               hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
 hipError_t launch_down_mfma(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream);
+// The same GEMMs on int8 MFMA with exact f64 sums, for few rows per expert: tiles of
+// i8_tile_rows rows, listed in i8_tiles (the f16 path's fixup list: at least two
+// entries per row, and every tile has a row).
+int i8_tile_rows(const LayerDesc& L, int T);
+inline int4* i8_tiles(const Workspace& ws) { return ws.fix; }
+hipError_t launch_gateup_i8(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream,
+                            hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
+hipError_t launch_down_i8(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream);
 // y_ssq (optional): y's RMSNorm partial sums, written with the rows (n_embd a
 // multiple of 32; otherwise ignored and left to the caller).
 hipError_t launch_combine(const LayerDesc& L, const Workspace& ws, int T, float* y, const float* residual,
                           hipStream_t stream, double* y_ssq = nullptr);
 // Decode sizes: token-major down projection with the combine in its epilogue
-// (replaces launch_experts_down + launch_combine when down_combine_fused()).
+// (replaces launch_down_i8 + launch_combine when down_combine_fused()).
 bool down_combine_fused(const LayerDesc& L, int T);
 // The token-per-workgroup down+combine kernel takes the layer's K + S steps.
 bool down_combine_tok_fits(const LayerDesc& L);

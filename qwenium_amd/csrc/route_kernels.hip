@@ -569,9 +569,20 @@ struct TopkArgs {
     int32_t* counters;    // [0] n_active, [1] n_tiles
     int4* tiles;
     int max_tiles;
+    int tile_shift;       // tiles of 1 << tile_shift rows
+    int sh_tiles_first;   // the shared expert's tiles before the routed experts' (else after them)
     int nblk;             // top-k blocks
     int tpb;              // tokens per top-k block (a wave each): 16, or 8 / 4 where fewer tokens fill the CUs
 };
+
+// Tiles of n rows, and tile i of the n rows of expert e from row off.
+__device__ __forceinline__ int n_row_tiles(const TopkArgs& a, int n) { return (n + (1 << a.tile_shift) - 1) >> a.tile_shift; }
+__device__ __forceinline__ int4 row_tile(const TopkArgs& a, int e, int off, int n, int i) {
+    return make_int4(e, off + (i << a.tile_shift), min(1 << a.tile_shift, n - (i << a.tile_shift)), 0);
+}
+// The routed experts' first tile, and the shared expert's with nr routed tiles.
+__device__ __forceinline__ int routed_tile0(const TopkArgs& a) { return a.sh_tiles_first && a.S ? n_row_tiles(a, a.T) : 0; }
+__device__ __forceinline__ int shared_tile0(const TopkArgs& a, int nr) { return a.sh_tiles_first ? 0 : nr; }
 
 constexpr int kMaxExpertsPerLane = 16;  // E <= 1024
 constexpr int kMaxTopK = 64;
@@ -1096,7 +1107,7 @@ __device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, const uint
         e = wave * 64 + lane;
         cnt = e < a.E ? s_cnt[e] : 0;
         act = cnt > 0 ? 1 : 0;
-        nt = (cnt + kMfmaTileM - 1) / kMfmaTileM;
+        nt = n_row_tiles(a, cnt);
         inc = wave_incl_scan_i32(cnt);
         inc_act = wave_incl_scan_i32(act);
         inc_t = wave_incl_scan_i32(nt);
@@ -1118,9 +1129,8 @@ __device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, const uint
                 a.slot_info[slot] = make_int4(e, off, cnt, first_token ? (int)__builtin_ctz(first_token[e]) : 0);
                 if (a.dslots && first_token) a.dslots[slot] = make_int4(e, off, cnt, (int)first_token[e]);
             }
-            const int tb = base_t + inc_t - nt;
-            for (int i = 0; i < nt && tb + i < a.max_tiles; ++i)
-                a.tiles[tb + i] = make_int4(e, off + i * kMfmaTileM, min(kMfmaTileM, cnt - i * kMfmaTileM), 0);
+            const int tb = routed_tile0(a) + base_t + inc_t - nt;
+            for (int i = 0; i < nt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, e, off, cnt, i);
         }
         if (wave == nchunk - 1 && a.dslots && first_token) {
             // decode slot list: the active routed experts, then "none" up to the
@@ -1139,9 +1149,9 @@ __device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, const uint
                 a.active[n_act] = a.E;
                 a.slot_info[n_act] = make_int4(a.E, A, a.T, 0);
                 n_act++;
-                const int ntt = (a.T + kMfmaTileM - 1) / kMfmaTileM;
-                for (int i = 0; i < ntt && n_tiles < a.max_tiles; ++i)
-                    a.tiles[n_tiles++] = make_int4(a.E, A + i * kMfmaTileM, min(kMfmaTileM, a.T - i * kMfmaTileM), 0);
+                const int ntt = n_row_tiles(a, a.T), tb = shared_tile0(a, n_tiles);
+                for (int i = 0; i < ntt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, a.E, A, a.T, i);
+                n_tiles += ntt;
             }
             a.counters[0] = n_act;
             a.counters[1] = n_tiles;
@@ -1167,22 +1177,22 @@ struct SmallRouteLds {
 
 // The expert scans of scan_experts (same tables) for the masks of at most 32
 // tokens, by one wave: lane l takes experts l * epl .. l * epl + epl - 1 in
-// order, three wave scans give each lane its bases.  Writes the offsets to
+// order, two wave scans give each lane its bases.  Writes the offsets to
 // s_off as well.
 static_assert(kTopkTokensPerBlock <= 32, "token masks are 32-bit");
 __device__ void scan_experts_wave(const TopkArgs& a, const uint32_t* mask, int32_t* s_off) {
     const int lane = threadIdx.x & 63;
     const int epl = (a.E + 63) >> 6;
     const int e0 = lane * epl, e1 = min(a.E, e0 + epl);
-    int c = 0, ac = 0, tc = 0;
+    int c = 0, ac = 0;
     for (int e = e0; e < e1; ++e) {
         const int n = __builtin_popcount(mask[e]);
         c += n;
         ac += n > 0 ? 1 : 0;
-        tc += (n + kMfmaTileM - 1) / kMfmaTileM;
     }
-    const int ic = wave_incl_scan_i32(c), ia = wave_incl_scan_i32(ac), it = wave_incl_scan_i32(tc);
-    int off = ic - c, slot = ia - ac, tile = it - tc;
+    const int ic = wave_incl_scan_i32(c), ia = wave_incl_scan_i32(ac);
+    int off = ic - c, slot = ia - ac;
+    const int t0 = routed_tile0(a);
     for (int e = e0; e < e1; ++e) {
         const uint32_t m = mask[e];
         const int n = __builtin_popcount(m);
@@ -1194,10 +1204,7 @@ __device__ void scan_experts_wave(const TopkArgs& a, const uint32_t* mask, int32
             a.expert_slot[e] = slot;
             a.slot_info[slot] = make_int4(e, off, n, (int)__builtin_ctz(m));
             if (a.dslots) a.dslots[slot] = make_int4(e, off, n, (int)m);
-            const int nt = (n + kMfmaTileM - 1) / kMfmaTileM;
-            for (int i = 0; i < nt && tile + i < a.max_tiles; ++i)
-                a.tiles[tile + i] = make_int4(e, off + i * kMfmaTileM, min(kMfmaTileM, n - i * kMfmaTileM), 0);
-            tile += nt;
+            if (a.tiles && t0 + slot < a.max_tiles) a.tiles[t0 + slot] = make_int4(e, off, n, 0);  // at most 16 rows: one tile
             ++slot;
         }
         off += n;
@@ -1212,16 +1219,16 @@ __device__ void scan_experts_wave(const TopkArgs& a, const uint32_t* mask, int32
     }
     if (lane == 0) {
         int n_act = n_routed;
-        int n_tiles = __builtin_amdgcn_readlane(it, 63);
+        int n_tiles = n_routed;
         a.offsets[a.E] = A;
         a.offsets[a.E + 1] = A + a.S * a.T;
         if (a.S) {
             a.active[n_act] = a.E;
             a.slot_info[n_act] = make_int4(a.E, A, a.T, 0);
             n_act++;
-            const int ntt = (a.T + kMfmaTileM - 1) / kMfmaTileM;
-            for (int i = 0; i < ntt && n_tiles < a.max_tiles; ++i)
-                a.tiles[n_tiles++] = make_int4(a.E, A + i * kMfmaTileM, min(kMfmaTileM, a.T - i * kMfmaTileM), 0);
+            const int ntt = n_row_tiles(a, a.T), tb = shared_tile0(a, n_tiles);
+            for (int i = 0; a.tiles && i < ntt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, a.E, A, a.T, i);
+            n_tiles += ntt;
         }
         a.counters[0] = n_act;
         a.counters[1] = n_tiles;
@@ -1645,7 +1652,7 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
         if (i < e) {
             below += c;
             below_act += c > 0 ? 1 : 0;
-            below_t += (c + kMfmaTileM - 1) / kMfmaTileM;
+            below_t += n_row_tiles(a, c);
         }
     }
     int here = 0;
@@ -1692,9 +1699,9 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
                 a.active[n_act] = a.E;
                 a.slot_info[n_act] = make_int4(a.E, A, a.T, 0);
                 n_act++;
-                const int ntt = (a.T + kMfmaTileM - 1) / kMfmaTileM;
-                for (int i = 0; i < ntt && n_tiles < a.max_tiles; ++i)
-                    a.tiles[n_tiles++] = make_int4(a.E, A + i * kMfmaTileM, min(kMfmaTileM, a.T - i * kMfmaTileM), 0);
+                const int ntt = n_row_tiles(a, a.T), tb = shared_tile0(a, n_tiles);
+                for (int i = 0; i < ntt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, a.E, A, a.T, i);
+                n_tiles += ntt;
             }
             a.counters[0] = n_act;
             a.counters[1] = n_tiles;
@@ -1704,9 +1711,9 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
     }
     if (tid == 0) a.offsets[e] = off;
     if (cnt == 0) return;
-    const int nt = (cnt + kMfmaTileM - 1) / kMfmaTileM;
-    for (int i = tid; i < nt && tb + i < a.max_tiles; i += kListThreads)
-        a.tiles[tb + i] = make_int4(e, off + i * kMfmaTileM, min(kMfmaTileM, cnt - i * kMfmaTileM), 0);
+    const int nt = n_row_tiles(a, cnt);
+    tb += routed_tile0(a);
+    for (int i = tid; i < nt && tb + i < a.max_tiles; i += kListThreads) a.tiles[tb + i] = row_tile(a, e, off, cnt, i);
     if (tid == 0) {
         a.active[slot] = e;
         a.expert_slot[e] = slot;
@@ -1834,7 +1841,7 @@ static hipError_t launch_router_exact(const LayerDesc& L, const Workspace& ws, c
 
 static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, const float* x, const float* xr, int T,
                                       const RouteDebug& dbg, bool& x_f16, hipStream_t stream, const float* norm_w,
-                                      float eps, const double* x_ssq) {
+                                      float eps, const double* x_ssq, int tile_rows) {
     TopkArgs ta;
     ta.norm_w = nullptr;
     ta.x_ssq = nullptr;
@@ -1871,8 +1878,11 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
     ta.expert_counts = L.expert_counts;
     ta.defer_softmax = 0;
     ta.counters = ws.counters;
-    ta.tiles = ws.tiles;
-    ta.max_tiles = ws.max_tiles;
+    ta.tiles = tile_rows == kMfmaTileM ? ws.tiles : i8_tiles(ws);
+    ta.max_tiles = tile_rows == kMfmaTileM ? ws.max_tiles : ws.fix_max;
+    ta.tile_shift = __builtin_ctz((unsigned)tile_rows);
+    ta.sh_tiles_first = tile_rows != kMfmaTileM;
+    if (gateup_q_fused(L, T)) ta.tiles = nullptr;  // the decode slot list is read instead
     // the merged top-k keeps 16 tokens per block; otherwise blocks of 8 or 4 tokens
     // where blocks of 16 would leave CUs idle (a block's tokens run one after another
     // on its four SIMDs)
@@ -2022,13 +2032,13 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
 bool route_norm_fused(const LayerDesc& L, int T) { return route_decode_fused(L, T) && L.H <= 8 * kRdSlab; }
 
 hipError_t launch_route(const LayerDesc& L, const Workspace& ws, const float* x, const float* xr, int T,
-                        const RouteDebug& dbg, bool x_f16, hipStream_t stream, const float* norm_w, float eps,
-                        const double* x_ssq) {
+                        const RouteDebug& dbg, bool x_f16, int tile_rows, hipStream_t stream, const float* norm_w,
+                        float eps, const double* x_ssq) {
     // norm_w: decode routing (route_norm_fused, no f16 operands) or the batched
-    // router (its preparation writes the f16 operands), with x == xr
-    if (norm_w && (x != xr || (route_uses_mfma(L, T) ? !x_f16 : (x_f16 || !route_norm_fused(L, T)))))
+    // router (its preparation writes every operand), with x == xr
+    if (norm_w && (x != xr || (!route_uses_mfma(L, T) && (x_f16 || !route_norm_fused(L, T)))))
         return hipErrorInvalidValue;
-    hipError_t err = launch_route_tables(L, ws, x, xr, T, dbg, x_f16, stream, norm_w, eps, x_ssq);
+    hipError_t err = launch_route_tables(L, ws, x, xr, T, dbg, x_f16, stream, norm_w, eps, x_ssq, tile_rows);
     if (err != hipSuccess || !x_f16) return err;
     // the routing launch did not write x's f16 quants (only the batched router's does)
     hipLaunchKernelGGL(k_x_f16, dim3((T + 3) / 4), dim3(256), 0, stream, x, T, L.H, ws.x_q, ws.x_d, ws.xq_qs, ws.xq_ds);

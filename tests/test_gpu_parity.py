@@ -889,3 +889,49 @@ def test_python_checks_on_device_operands(gpu):
     got = layer.forward(x, residual=res, workspace=ws, stream=s)
     s.synchronize()
     assert torch.equal(got, want)
+
+
+# ---- int8-MFMA expert GEMMs (17 tokens to the f16 path) ------------------------------------
+@pytest.mark.parametrize("wtype", [TYPE_Q4_0, TYPE_Q8_0])
+@pytest.mark.parametrize("hidden,ffn", [(256, 64), (512, 192), (768, 704), (1280, 576)])
+@pytest.mark.parametrize("experts,top_k,T", [
+    (1, 1, 17), (1, 1, 31), (1, 1, 32), (1, 1, 33), (1, 1, 129),  # all rows on one expert: 32-row tiles and their remainders
+    (16, 2, 17), (16, 2, 40), (16, 2, 112), (16, 2, 113),         # 1 to ~20 rows: every group of four, both tile heights
+])
+def test_i8_experts_tile_edges(gpu, monkeypatch, wtype, hidden, ffn, experts, top_k, T):
+    """Tiles of 16 and 32 rows with every remainder, reduction lengths that end in a partial
+    chunk (Q4_0 chunks of 8 block pairs, Q8_0 of 4: 1 to 11 pairs here) and ffn widths of odd
+    column groups: routing bit-exact, h quants and outputs bit-identical to the oracle's (the
+    sums are exact in f64 on both sides)."""
+    monkeypatch.setenv("QMOE_MFMA_MIN_TOKENS", "100000")
+    spec = LayerSpec(hidden, experts, top_k, ffn, True, wtype)
+    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=300 + T + hidden)
+    assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0)
+
+
+def test_i8_experts_gate_up_strides(gpu):
+    """Gate and up rows of different strides (views into wider rows): the int8 GEMM's two
+    column bases; equal to the packed layer's results bit for bit."""
+    from qwenium_amd import GGMLTensor
+
+    class Strided(GGMLTensor):
+        def desc(self):
+            d = super().desc()
+            d.nb[1] = self.data.shape[1]
+            d.nb[2] = d.nb[1] * self.ne[1]
+            return d
+
+    spec = LayerSpec(512, 8, 2, 128, False, TYPE_Q4_0)
+    tensors = synthetic.make_layer_tensors(spec, 11)
+    x = synthetic.make_x(spec, 50, 11)
+    y = synthetic.make_layer(spec, 11, tensors=tensors).forward(x)
+    wide = dict(tensors)
+    for name, pad in (("gate", 36), ("up", 92)):
+        t = tensors[name]
+        rows = t.data.view(8 * 128, -1)
+        buf = torch.full((rows.shape[0], rows.shape[1] + pad), 0x7f, dtype=torch.uint8, device=rows.device)
+        buf[:, :rows.shape[1]] = rows
+        wide[name] = Strided(buf, t.type, t.ne)
+    y2 = synthetic.make_layer(spec, 11, tensors=wide, prefill_copies=False).forward(x)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2)
