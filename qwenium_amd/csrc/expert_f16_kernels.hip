@@ -78,7 +78,14 @@ static_assert(kNM == 4, "the main loop instantiates 1..4 row tiles");
 constexpr int kScaleBytes = kTM * 16;       // per row and chunk: its 4 f16 block scales, twice
 constexpr int kStageBytes = kAHalfs * 2 + kScaleBytes;
 constexpr int kHLd = 64 + 4;                // gate/up epilogue: g and u rows in LDS, f32
-constexpr size_t kF16LdsBytes = 2 * (size_t)kStageBytes + kSinkBytes + kTM * 8;
+// Q8_0: this thread's staging offsets live in LDS.  Its weights take ten registers
+// more than Q4_0's; spilled, the offsets' reloads waited for every load before them
+// (layer at 2048 tokens of skewed routing: 595 us so, 512 with twelve spills in the
+// fully staged form, 470 from LDS)
+constexpr int kOffSlots = kDmaIters + kScaleRounds;
+template <int WT> constexpr bool kOffLds = WT == kTypeQ8_0;
+template <int WT>
+constexpr size_t kF16LdsBytes = 2 * (size_t)kStageBytes + kSinkBytes + kTM * 8 + (kOffLds<WT> ? (size_t)kOffSlots * 256 * 4 : 0);
 static_assert(2 * 64 * kHLd * 4 <= 2 * (size_t)kStageBytes, "an epilogue pass's g and u rows fit the stage buffers");
 // Error model of the gate/up epilogue's f32 values.  The accumulation error of
 // g (n block terms summed by fma in f32) relative to max(|g|, rms of the
@@ -410,6 +417,7 @@ __global__ __launch_bounds__(256, 3) void k_expert_f16(F16Args a) {
     uint8_t* s_stage = s_dyn;
     uint32_t* s_rowoff = (uint32_t*)(s_dyn + 2 * kStageBytes + kSinkBytes);
     uint32_t* s_doff = s_rowoff + kTM;
+    uint32_t* s_off = s_doff + kTM;  // kOffLds: [kOffSlots][256]
     // XCD-aware mapping (workgroups are dealt to the 8 XCDs round-robin): XCD x
     // takes tiles x, x + 8, ... and all column chunks of each, so a tile's
     // activation rows are read into one L2 and the XCDs get statistically
@@ -429,6 +437,7 @@ __global__ __launch_bounds__(256, 3) void k_expert_f16(F16Args a) {
     const bool sh = e >= a.E;
     const int nm = (nr + 31) >> 5;  // 32-row MFMA tiles with rows (wave-uniform)
     const int nblk = a.K >> 5;
+    const int slots_nm = 32 * nm * kSlotsPerRow;  // the staging slots of those tiles' rows
 
     if (tid < kTM) {
         const int pr = p0 + min(tid, nr - 1);
@@ -476,6 +485,7 @@ __global__ __launch_bounds__(256, 3) void k_expert_f16(F16Args a) {
         const int r = s / kSlotsPerRow;
         const int u = s - r * kSlotsPerRow;
         soff[it] = s_rowoff[r] + (u < kSlotsPerRow - 1 ? 8 * u : 0);
+        if (kOffLds<WT>) s_off[it * 256 + tid] = soff[it];
     }
     // Scales: each row's 16-byte record holds the chunk's block scales: with
     // 128-wide chunks its 4 scales twice (dword d = blocks 2 (d & 1), + 1), with
@@ -487,23 +497,29 @@ __global__ __launch_bounds__(256, 3) void k_expert_f16(F16Args a) {
     for (int rd = 0; rd < kScaleRounds; ++rd) {
         const int sl = 256 * rd + wave * 64 + lane;
         doff[rd] = s_doff[sl >> 2] + (kPPC == 2 ? 2 * (sl & 1) : 0);
+        if (kOffLds<WT>) s_off[(kDmaIters + rd) * 256 + tid] = doff[rd];
     }
+    // Only the row tiles that have rows are staged (an expert's last tile holds 64 of
+    // 128 rows on average): Gemma 4 layer at 1500 tokens 514 -> 457 us.
     auto stage = [&](int c, int buf) {
         uint8_t* st = s_stage + buf * kStageBytes;
         const uint32_t k0 = (uint32_t)(c * kKC);
 #pragma unroll
         for (int it = 0; it < kDmaIters; ++it) {
             const int s0 = it * 256 + wave * 64;
+            if (s0 >= slots_nm) break;  // (wave-uniform)
             const void* dst = s0 < kASlots ? (const void*)(st + s0 * 16) : (const void*)(s_stage + 2 * kStageBytes);
-            dma_lds16(a.a_q + k0, 2u * soff[it], __builtin_amdgcn_readfirstlane(lds_addr(dst)));  // wave-uniform
+            dma_lds16(a.a_q + k0, 2u * (kOffLds<WT> ? s_off[it * 256 + tid] : soff[it]), __builtin_amdgcn_readfirstlane(lds_addr(dst)));  // wave-uniform
         }
         // a 2-block last chunk: the odd dwords (blocks 2, 3, past the row) reload
         // blocks 0, 1, so every scale the MFMA multiplies (by 0 or not) is finite
         const uint32_t back = (kPPC == 2 && 4 * c + 4 > nblk && (lane & 1)) ? 4u : 0u;
 #pragma unroll
-        for (int rd = 0; rd < kScaleRounds; ++rd)
-            dma_lds4(a.a_d + 2 * kPPC * c, 2u * doff[rd] - back,
+        for (int rd = 0; rd < kScaleRounds; ++rd) {
+            if (rd * 64 >= 32 * nm) break;
+            dma_lds4(a.a_d + 2 * kPPC * c, 2u * (kOffLds<WT> ? s_off[(kDmaIters + rd) * 256 + tid] : doff[rd]) - back,
                      __builtin_amdgcn_readfirstlane(lds_addr(st + kAHalfs * 2 + (256 * rd + wave * 64) * 4)));
+        }
     };
 
     v16f acc[kNM];
@@ -847,13 +863,14 @@ static F16Args base_f16_args(const LayerDesc& L, const Workspace& ws) {
     return a;
 }
 
-template <typename Kern>
-static hipError_t launch_f16(Kern kern, dim3 grid, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop,
-                             const F16Args& a) {
+template <int WT, bool GATEUP, int ACT>
+static hipError_t launch_f16(dim3 grid, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop, const F16Args& a) {
+    const auto kern = k_expert_f16<WT, GATEUP, ACT>;
+    constexpr size_t lds = kF16LdsBytes<WT>;
     // above the 64 KiB default dynamic LDS window: raise it (idempotent)
-    hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kF16LdsBytes);
+    hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return err;
-    launch_timed(kern, grid, dim3(256), kF16LdsBytes, stream, ev_start, ev_stop, a);
+    launch_timed(kern, grid, dim3(256), lds, stream, ev_start, ev_stop, a);
     return hipGetLastError();
 }
 
@@ -873,11 +890,11 @@ hipError_t launch_gateup_mfma(const LayerDesc& L, const Workspace& ws, int T, hi
     const dim3 grid(8 * ((std::min(ws.max_tiles, max_row_tiles(L, T, kTM)) + 7) / 8) * a.n_y);
     const bool gelu = L.act == kActGeluTanh;
     if (L.gu_type == kTypeQ4_0)
-        err = gelu ? launch_f16(k_expert_f16<kTypeQ4_0, true, kActGeluTanh>, grid, stream, ev_start, ev_stop, a)
-                   : launch_f16(k_expert_f16<kTypeQ4_0, true, kActSilu>, grid, stream, ev_start, ev_stop, a);
+        err = gelu ? launch_f16<kTypeQ4_0, true, kActGeluTanh>(grid, stream, ev_start, ev_stop, a)
+                   : launch_f16<kTypeQ4_0, true, kActSilu>(grid, stream, ev_start, ev_stop, a);
     else
-        err = gelu ? launch_f16(k_expert_f16<kTypeQ8_0, true, kActGeluTanh>, grid, stream, ev_start, ev_stop, a)
-                   : launch_f16(k_expert_f16<kTypeQ8_0, true, kActSilu>, grid, stream, ev_start, ev_stop, a);
+        err = gelu ? launch_f16<kTypeQ8_0, true, kActGeluTanh>(grid, stream, ev_start, ev_stop, a)
+                   : launch_f16<kTypeQ8_0, true, kActSilu>(grid, stream, ev_start, ev_stop, a);
     if (err != hipSuccess) return err;
     FixArgs f{};
     f.H = L.H; f.F = L.F; f.E = L.E;
@@ -906,8 +923,8 @@ hipError_t launch_down_mfma(const LayerDesc& L, const Workspace& ws, int T, hipS
     a.K = L.F;
     a.n_y = L.H / 128;
     const dim3 grid(8 * ((std::min(ws.max_tiles, max_row_tiles(L, T, kTM)) + 7) / 8) * a.n_y);
-    return L.dn_type == kTypeQ4_0 ? launch_f16(k_expert_f16<kTypeQ4_0, false, kActSilu>, grid, stream, nullptr, nullptr, a)
-                                  : launch_f16(k_expert_f16<kTypeQ8_0, false, kActSilu>, grid, stream, nullptr, nullptr, a);
+    return L.dn_type == kTypeQ4_0 ? launch_f16<kTypeQ4_0, false, kActSilu>(grid, stream, nullptr, nullptr, a)
+                                  : launch_f16<kTypeQ8_0, false, kActSilu>(grid, stream, nullptr, nullptr, a);
 }
 
 }  // namespace qmoe
