@@ -24,12 +24,8 @@ struct ExpertArgs {
     const uint8_t* w_down; uint64_t down_nb1, down_nb2;
     const uint8_t* w_sh_gate; const uint8_t* w_sh_up; const uint8_t* w_sh_down;
     uint64_t sh_gate_nb1, sh_up_nb1, sh_down_nb1;
-    const int32_t* counters;   // [0] n_active
-    const int4* slot_info;     // [E+1] {expert, first row, rows, token of first row}
-    const int32_t* offsets;    // [E+2]
     const int32_t* row_token;  // [R]
     const int8_t* xq_qs; const float2* xq_ds;  // [T][H], [T][H/32]
-    float2* gubuf;                             // [R][F] (gate, up) projections (f32)
     int8_t* hq_qs; float2* hq_ds;              // [R][F], [R][F/32] Q8_0 of hbuf
     float* ybuf;                               // [R][H] down outputs (unweighted)
     int act;                                   // kActSilu or kActGeluTanh
@@ -559,8 +555,8 @@ static ExpertArgs make_expert_args(const LayerDesc& L, const Workspace& ws, int 
     a.w_down = L.w_down; a.down_nb1 = L.down_nb1; a.down_nb2 = L.down_nb2;
     a.w_sh_gate = L.w_sh_gate; a.w_sh_up = L.w_sh_up; a.w_sh_down = L.w_sh_down;
     a.sh_gate_nb1 = L.sh_gate_nb1; a.sh_up_nb1 = L.sh_up_nb1; a.sh_down_nb1 = L.sh_down_nb1;
-    a.counters = ws.counters; a.slot_info = ws.slot_info; a.offsets = ws.offsets; a.row_token = ws.row_token;
-    a.xq_qs = ws.xq_qs; a.xq_ds = ws.xq_ds; a.gubuf = ws.gubuf; a.hq_qs = ws.hq_qs; a.hq_ds = ws.hq_ds;
+    a.row_token = ws.row_token;
+    a.xq_qs = ws.xq_qs; a.xq_ds = ws.xq_ds; a.hq_qs = ws.hq_qs; a.hq_ds = ws.hq_ds;
     a.ybuf = ws.ybuf;
     a.act = L.act;
     a.gelu_tab = L.gelu_tab;

@@ -152,9 +152,6 @@ size_t workspace_bytes(int T, int H, int E, int K, int F, Workspace* w, void* ba
     ws.rows = (int32_t*)take(R * sizeof(int32_t));
     ws.row_token = (int32_t*)take(R * sizeof(int32_t));
     ws.pos = (int32_t*)take(A * sizeof(int32_t));
-    ws.active = (int32_t*)take((size_t)(E + 1) * sizeof(int32_t));
-    ws.expert_slot = (int32_t*)take((size_t)E * sizeof(int32_t));
-    ws.slot_info = (int4*)take((size_t)(E + 1) * sizeof(int4));
     ws.dslots = (int4*)take((size_t)(E + 2) * sizeof(int4));
     ws.counters = (int32_t*)take(qmoe::kCounters * sizeof(int32_t));
     ws.sync = (int32_t*)take(kSyncWords * sizeof(int32_t));

@@ -28,8 +28,7 @@ constexpr int kRmsMaxChunks = 256;
 constexpr int kMfmaTileM = 128;
 // k values per LDS chunk of the prefill GEMMs.
 constexpr int kF16ChunkK = 64;
-// Workspace counters (kCounters ints): [0] active slots, [1] tiles,
-// [kCounterFix] listed h blocks.
+// Workspace counters (kCounters ints): [1] tiles, [kCounterFix] listed h blocks.
 constexpr int kCounters = 32;
 constexpr int kCounterFix = 4;
 constexpr int kFixStride = 36;  // floats per listed h block: 32 values, amax's error estimate, padding
@@ -96,21 +95,18 @@ struct Workspace {
     int32_t* rows = nullptr;      // [R] assignment id (t*K+j); shared rows: -1
     int32_t* row_token = nullptr; // [R]
     int32_t* pos = nullptr;       // [T*K] position of assignment
-    int32_t* active = nullptr;    // [E+1] active experts (ascending), shared (=E) last
-    int32_t* expert_slot = nullptr; // [E] slot of each active expert
-    int4* slot_info = nullptr;    // [E+1] per active slot {expert, first row, rows, 0}
     int4* dslots = nullptr;       // [E+2] decode slot list {expert, first row, rows, token mask}:
                                   // active routed experts, then expert -1 up to min(E, T*K)
-    int32_t* counters = nullptr;  // [kCounters] n_active, n_tiles, ...
+    int32_t* counters = nullptr;  // [kCounters]
     int32_t* sync = nullptr;      // [kSyncWords] zeroed at creation: the merged top-k's finished-workgroup counter
     int4* tiles = nullptr;        // [max tiles] {expert, row0, nrows, 0}
-    float2* gubuf = nullptr;      // [R][F] (gate, up) projections
+    float2* gubuf = nullptr;      // [R][F] the room of h_q
     int8_t* hq_qs = nullptr;      // [R][F]   Q8_0 quants of h = silu(g)*u
     float2* hq_ds = nullptr;      // [R][F/32] {d, bitcast(sum q)}
     // prefill GEMM operands: Q8_0 quants as exact f16 values and fp16 block scales
     _Float16* x_q = nullptr;      // [T][H] x (the experts' input)
     uint16_t* x_d = nullptr;      // [T][H/32]
-    _Float16* h_q = nullptr;      // [R][F] h (aliases gubuf: the prefill path writes no (g, u))
+    _Float16* h_q = nullptr;      // [R][F] h (in gubuf)
     uint16_t* h_d = nullptr;      // [R][F/32]
     // batched router operands: bf16 hi/lo splits of the router input and weights, row norms
     uint16_t* rx_split = nullptr; // [2][T][H] (hi, lo)

@@ -560,13 +560,10 @@ struct TopkArgs {
     int32_t* rows;        // [R]
     int32_t* row_token;   // [R]
     int32_t* pos;         // [T*K]
-    int32_t* active;      // [E+1]
-    int32_t* expert_slot; // [E]
-    int4* slot_info;      // [E+1] {expert, first row, rows, token of first row}
     int4* dslots;         // [E+2] decode slot list (decode routing only, else null)
     unsigned long long* expert_counts;  // optional [E]: per-expert dispatch counts accumulated
     int defer_softmax;    // 1: the selection leaves the softmax to the caller (token_softmax)
-    int32_t* counters;    // [0] n_active, [1] n_tiles
+    int32_t* counters;    // [1] n_tiles, [kCounterFix]
     int4* tiles;
     int max_tiles;
     int tile_shift;       // tiles of 1 << tile_shift rows
@@ -977,8 +974,7 @@ static inline int topk_epl(int E) {
     return epl <= 1 ? 1 : epl <= 2 ? 2 : epl <= 4 ? 4 : epl <= 8 ? 8 : 16;
 }
 
-__device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, const uint32_t* first_token, int32_t* s_off,
-                             int32_t* s_misc);
+__device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, int32_t* s_off, int32_t* s_misc);
 
 // blockDim = 64 * a.tpb: one wave per token.  Writes the selection and, per
 // expert, the mask of the block's tokens that chose it.
@@ -1058,34 +1054,54 @@ __global__ __launch_bounds__(64 * kTopkTokensPerBlock) void k_topk(TopkArgs a, i
         __syncthreads();
         if (!s_last) return;
         if (tid == 0) __hip_atomic_store(sync + kSyncTopk, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // per expert: the blocks' bases (exclusive prefix of their counts) and the total
+        // what the scatter reads of this thread's first two assignments, requested with
+        // the counts below
+        const int A = a.T * a.K;
+        constexpr int kAhead = 2;
+        int ex_n[kAhead], rank_n[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const int i = min(tid + k * (int)blockDim.x, A - 1);
+            ex_n[k] = __hip_atomic_load(a.topk_idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            rank_n[k] = __hip_atomic_load(a.local_rank + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        // per expert: the blocks' bases (exclusive prefix of their counts) and the total,
+        // eight counts in flight (one after another each waits a trip past the L2s: the
+        // launch 13.8 -> 11.9 us at 14 blocks, 10.4 -> 9.3 at 4)
         for (int e = tid; e < a.E; e += blockDim.x) {
             int run = 0;
-            for (int b = 0; b < (int)gridDim.x; ++b) {
-                const int c = __hip_atomic_load(a.hist + (uint64_t)b * a.E + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s_base[b * a.E + e] = run;
-                run += c;
+            for (int b0 = 0; b0 < (int)gridDim.x; b0 += 8) {
+                int c[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    c[k] = __hip_atomic_load(a.hist + (uint64_t)min(b0 + k, (int)gridDim.x - 1) * a.E + e, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    if (b0 + k < (int)gridDim.x) {
+                        s_base[(b0 + k) * a.E + e] = run;
+                        run += c[k];
+                    }
             }
             s_cnt[e] = run;
         }
         __syncthreads();
-        scan_experts(a, s_cnt, nullptr, s_off, s_misc);
+        scan_experts(a, s_cnt, s_off, s_misc);
         __syncthreads();
         // the stable scatter: assignment i of expert e to row offsets[e] + its block's
-        // base + its rank in the block; the first row's token into the slot table;
-        // the shared expert's rows in token order
-        const int A = a.T * a.K;
-        for (int i = tid; i < A + a.S * a.T; i += blockDim.x) {
+        // base + its rank in the block; the shared expert's rows in token order
+        int k = 0;
+        for (int i = tid; i < A + a.S * a.T; i += blockDim.x, ++k) {
             if (i < A) {
                 const int t = i / a.K;
-                const int ex = __hip_atomic_load(a.topk_idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const int off = s_off[ex];
-                const int p = off + s_base[(t / a.tpb) * a.E + ex] +
-                              __hip_atomic_load(a.local_rank + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int ex = k == 0 ? ex_n[0] : k == 1 ? ex_n[1]
+                                      : __hip_atomic_load(a.topk_idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int rank = k == 0 ? rank_n[0] : k == 1 ? rank_n[1]
+                                        : __hip_atomic_load(a.local_rank + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int p = s_off[ex] + s_base[(t / a.tpb) * a.E + ex] + rank;
                 a.rows[p] = i;
                 a.row_token[p] = t;
                 a.pos[i] = p;
-                if (p == off) ((int*)(a.slot_info + a.expert_slot[ex]))[3] = t;
             } else {
                 a.rows[i] = -1;
                 a.row_token[i] = i - A;
@@ -1094,66 +1110,42 @@ __global__ __launch_bounds__(64 * kTopkTokensPerBlock) void k_topk(TopkArgs a, i
     }
 }
 
-// Exclusive scans over experts of the per-expert counts in s_cnt: offsets,
-// active slots, expert->slot map, MFMA tiles, counters.  In one block of at
-// least E threads rounded to waves (E <= 1024).  first_token (optional, LDS)
-// gives the token of each expert's first row; otherwise the scatter sets it.
-__device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, const uint32_t* first_token,
-                             int32_t* s_off, int32_t* s_misc) {
+// Exclusive scans over experts of the per-expert counts in s_cnt: offsets, MFMA
+// tiles, counters.  In one block of at least E threads rounded to waves (E <= 1024).
+__device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, int32_t* s_off, int32_t* s_misc) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int nchunk = (a.E + 63) >> 6;
-    int cnt = 0, act = 0, nt = 0, inc = 0, inc_act = 0, inc_t = 0, e = 0;
+    int cnt = 0, nt = 0, inc = 0, inc_t = 0, e = 0;
     if (wave < nchunk) {
         e = wave * 64 + lane;
         cnt = e < a.E ? s_cnt[e] : 0;
-        act = cnt > 0 ? 1 : 0;
         nt = n_row_tiles(a, cnt);
         inc = wave_incl_scan_i32(cnt);
-        inc_act = wave_incl_scan_i32(act);
         inc_t = wave_incl_scan_i32(nt);
-        if (lane == 63) { s_misc[3 * wave] = inc; s_misc[3 * wave + 1] = inc_act; s_misc[3 * wave + 2] = inc_t; }
+        if (lane == 63) { s_misc[2 * wave] = inc; s_misc[2 * wave + 1] = inc_t; }
     }
     __syncthreads();
     if (wave < nchunk) {
-        int base = 0, base_act = 0, base_t = 0;
-        for (int w = 0; w < wave; ++w) { base += s_misc[3 * w]; base_act += s_misc[3 * w + 1]; base_t += s_misc[3 * w + 2]; }
+        int base = 0, base_t = 0;
+        for (int w = 0; w < wave; ++w) { base += s_misc[2 * w]; base_t += s_misc[2 * w + 1]; }
         if (e < a.E) {
             const int off = base + inc - cnt;
             a.offsets[e] = off;
-            if (s_off) s_off[e] = off;
-            if (act) {
-                const int slot = base_act + inc_act - 1;
-                if (a.expert_counts) atomicAdd(a.expert_counts + e, (unsigned long long)cnt);
-                a.active[slot] = e;
-                a.expert_slot[e] = slot;
-                a.slot_info[slot] = make_int4(e, off, cnt, first_token ? (int)__builtin_ctz(first_token[e]) : 0);
-                if (a.dslots && first_token) a.dslots[slot] = make_int4(e, off, cnt, (int)first_token[e]);
-            }
+            s_off[e] = off;
+            if (cnt > 0 && a.expert_counts) atomicAdd(a.expert_counts + e, (unsigned long long)cnt);
             const int tb = routed_tile0(a) + base_t + inc_t - nt;
             for (int i = 0; i < nt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, e, off, cnt, i);
         }
-        if (wave == nchunk - 1 && a.dslots && first_token) {
-            // decode slot list: the active routed experts, then "none" up to the
-            // most a forward can have (the shared expert is not in it)
-            const int n_routed = __builtin_amdgcn_readlane(base_act + inc_act, 63);
-            const int max_v = min(a.E, a.T * a.K);
-            for (int i = n_routed + lane; i < max_v; i += 64) a.dslots[i] = make_int4(-1, 0, 0, 0);
-        }
         if (wave == nchunk - 1 && lane == 63) {
             const int A = a.T * a.K;
-            int n_act = base_act + inc_act;
             int n_tiles = base_t + inc_t;
             a.offsets[a.E] = A;
             a.offsets[a.E + 1] = A + a.S * a.T;
             if (a.S) {
-                a.active[n_act] = a.E;
-                a.slot_info[n_act] = make_int4(a.E, A, a.T, 0);
-                n_act++;
                 const int ntt = n_row_tiles(a, a.T), tb = shared_tile0(a, n_tiles);
                 for (int i = 0; i < ntt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, a.E, A, a.T, i);
                 n_tiles += ntt;
             }
-            a.counters[0] = n_act;
             a.counters[1] = n_tiles;
             a.counters[kCounterFix] = 0;  // the prefill gate/up's list of uncertain h blocks starts empty
         }
@@ -1162,9 +1154,8 @@ __device__ void scan_experts(const TopkArgs& a, const int32_t* s_cnt, const uint
 
 // Whole routing for T <= kTopkTokensPerBlock in ONE block of 1024 threads,
 // everything in LDS: top-k per token (one wave each), per-expert token masks,
-// then wave 0 alone (no further barrier): counts, offsets, active slots (with
-// the token of each slot's first row = lowest mask bit), tiles, and the stable
-// scatter (rank = earlier tokens in the expert's mask), while the other waves
+// then wave 0 alone (no further barrier): counts, offsets, the decode slot
+// list (or tiles), and the stable scatter (rank = earlier tokens in the expert's mask), while the other waves
 // run the deferred softmax.  Reads the exact logits from a.logits.
 struct SmallRouteLds {
     int32_t idx[kTopkTokensPerBlock][kMaxTopK];
@@ -1200,9 +1191,6 @@ __device__ void scan_experts_wave(const TopkArgs& a, const uint32_t* mask, int32
         s_off[e] = off;
         if (n > 0) {
             if (a.expert_counts) atomicAdd(a.expert_counts + e, (unsigned long long)n);
-            a.active[slot] = e;
-            a.expert_slot[e] = slot;
-            a.slot_info[slot] = make_int4(e, off, n, (int)__builtin_ctz(m));
             if (a.dslots) a.dslots[slot] = make_int4(e, off, n, (int)m);
             if (a.tiles && t0 + slot < a.max_tiles) a.tiles[t0 + slot] = make_int4(e, off, n, 0);  // at most 16 rows: one tile
             ++slot;
@@ -1218,19 +1206,14 @@ __device__ void scan_experts_wave(const TopkArgs& a, const uint32_t* mask, int32
         for (int i = n_routed + lane; i < max_v; i += 64) a.dslots[i] = make_int4(-1, 0, 0, 0);
     }
     if (lane == 0) {
-        int n_act = n_routed;
         int n_tiles = n_routed;
         a.offsets[a.E] = A;
         a.offsets[a.E + 1] = A + a.S * a.T;
         if (a.S) {
-            a.active[n_act] = a.E;
-            a.slot_info[n_act] = make_int4(a.E, A, a.T, 0);
-            n_act++;
             const int ntt = n_row_tiles(a, a.T), tb = shared_tile0(a, n_tiles);
             for (int i = 0; a.tiles && i < ntt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, a.E, A, a.T, i);
             n_tiles += ntt;
         }
-        a.counters[0] = n_act;
         a.counters[1] = n_tiles;
         a.counters[kCounterFix] = 0;
     }
@@ -1608,16 +1591,16 @@ __global__ __launch_bounds__(1024) void k_route_decode_tables(TopkArgs a, int8_t
 // The expert lists from the top-k blocks' token masks, one workgroup per
 // expert and one more (index E) for the shared expert's rows and the totals.
 // The top-k blocks added their counts into the per-expert totals, so each
-// workgroup finds its expert's first row, active slot and first tile by
+// workgroup finds its expert's first row and first tile by
 // summing the totals below it, and none waits for another.  It then scans its
 // column of masks (threads own consecutive blocks) and writes the expert's rows
-// in token order: the same offsets, slots, tiles, rows and positions as
+// in token order: the same offsets, tiles, rows and positions as
 // scan_experts followed by the stable scatter.
 constexpr int kListThreads = 256;
 constexpr int kListRegs = 4;  // masks per thread held in registers (nblk <= 1024); beyond, loaded twice
 
 __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
-    __shared__ int32_t s_red[3][kListThreads / 64];
+    __shared__ int32_t s_red[2][kListThreads / 64];
     __shared__ int32_t s_wtot[kListThreads / 64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int e = (int)blockIdx.x;
@@ -1640,8 +1623,8 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
             if (jslot) js[i] = a.jslot[h];
         }
     }
-    // rows, active experts and tiles of the experts below e (all of them for e = E)
-    int below = 0, below_act = 0, below_t = 0;
+    // rows and tiles of the experts below e (all of them for e = E)
+    int below = 0, below_t = 0;
     for (int i = tid; i < a.E; i += kListThreads) {
         int cp[kTotalCopies];
 #pragma unroll
@@ -1651,7 +1634,6 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
         for (int r = 0; r < kTotalCopies; ++r) c += cp[r];
         if (i < e) {
             below += c;
-            below_act += c > 0 ? 1 : 0;
             below_t += n_row_tiles(a, c);
         }
     }
@@ -1663,47 +1645,39 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         below += __shfl_xor(below, o, 64);
-        below_act += __shfl_xor(below_act, o, 64);
         below_t += __shfl_xor(below_t, o, 64);
     }
     const int inc = wave_incl_scan_i32(here);
     if (lane == 63) s_wtot[wave] = inc;
     if (lane == 0) {
         s_red[0][wave] = below;
-        s_red[1][wave] = below_act;
-        s_red[2][wave] = below_t;
+        s_red[1][wave] = below_t;
     }
     __syncthreads();
-    int off = 0, slot = 0, tb = 0, wbase = 0, cnt = 0;
+    int off = 0, tb = 0, wbase = 0, cnt = 0;
 #pragma unroll
     for (int w = 0; w < kListThreads / 64; ++w) {
         off += s_red[0][w];
-        slot += s_red[1][w];
-        tb += s_red[2][w];
+        tb += s_red[1][w];
         wbase += w < wave ? s_wtot[w] : 0;
         cnt += s_wtot[w];
     }
     if (!routed) {
-        // the shared expert's rows in token order, the slot and tile totals, the counters
+        // the shared expert's rows in token order and its tiles, the tile total, the counters
         const int A = a.T * a.K;
-        if (a.S)
+        int n_tiles = tb;
+        if (a.S) {
             for (int t = tid; t < a.T; t += kListThreads) {
                 a.rows[A + t] = -1;
                 a.row_token[A + t] = t;
             }
+            const int ntt = n_row_tiles(a, a.T), t0 = shared_tile0(a, n_tiles);
+            for (int i = tid; i < ntt && t0 + i < a.max_tiles; i += kListThreads) a.tiles[t0 + i] = row_tile(a, a.E, A, a.T, i);
+            n_tiles += ntt;
+        }
         if (tid == 0) {
-            int n_act = slot, n_tiles = tb;
             a.offsets[a.E] = A;
             a.offsets[a.E + 1] = A + a.S * a.T;
-            if (a.S) {
-                a.active[n_act] = a.E;
-                a.slot_info[n_act] = make_int4(a.E, A, a.T, 0);
-                n_act++;
-                const int ntt = n_row_tiles(a, a.T), tb = shared_tile0(a, n_tiles);
-                for (int i = 0; i < ntt && tb + i < a.max_tiles; ++i) a.tiles[tb + i] = row_tile(a, a.E, A, a.T, i);
-                n_tiles += ntt;
-            }
-            a.counters[0] = n_act;
             a.counters[1] = n_tiles;
             a.counters[kCounterFix] = 0;  // the prefill gate/up's list of uncertain h blocks starts empty
         }
@@ -1714,11 +1688,7 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
     const int nt = n_row_tiles(a, cnt);
     tb += routed_tile0(a);
     for (int i = tid; i < nt && tb + i < a.max_tiles; i += kListThreads) a.tiles[tb + i] = row_tile(a, e, off, cnt, i);
-    if (tid == 0) {
-        a.active[slot] = e;
-        a.expert_slot[e] = slot;
-        if (a.expert_counts) atomicAdd(a.expert_counts + e, (unsigned long long)cnt);
-    }
+    if (tid == 0 && a.expert_counts) atomicAdd(a.expert_counts + e, (unsigned long long)cnt);
     // this thread's rows start after the rows of the blocks before its own
     int p = off + wbase + inc - here;
     auto put = [&](int b, uint32_t m, uint64_t jw) {
@@ -1739,7 +1709,6 @@ __global__ __launch_bounds__(kListThreads) void k_lists(TopkArgs a) {
                 }
             }
             const int i = t * a.K + j;
-            if (p == off) a.slot_info[slot] = make_int4(e, off, cnt, t);
             a.rows[p] = i;
             a.row_token[p] = t;
             a.pos[i] = p;
@@ -1871,9 +1840,6 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
     ta.rows = ws.rows;
     ta.row_token = ws.row_token;
     ta.pos = ws.pos;
-    ta.active = ws.active;
-    ta.expert_slot = ws.expert_slot;
-    ta.slot_info = ws.slot_info;
     ta.dslots = nullptr;
     ta.expert_counts = L.expert_counts;
     ta.defer_softmax = 0;
