@@ -935,3 +935,25 @@ def test_i8_experts_gate_up_strides(gpu):
     y2 = synthetic.make_layer(spec, 11, tensors=wide, prefill_copies=False).forward(x)
     torch.cuda.synchronize()
     assert torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("H", [4, 32, 100, 256, 260, 2048, 2816, 4092, 4096])
+def test_norm_rows_aligned_equals_general(gpu, H):
+    """The one-pass RMSNorm and Gemma 4 input kernel of 16-byte aligned rows against the general
+    one (the same rows at an odd float offset): equal bits, at one thread, whole and partial
+    waves, and the widest row."""
+    from qwenium_amd import gemma4_moe_inputs, rms_norm
+
+    T = 3
+    x, w, w2 = (torch.randn(n, dtype=torch.float32, device="cuda") for n in (T * H, H, H))
+
+    def odd(v):
+        return torch.cat([v.new_zeros(1), v])[1:]
+
+    assert odd(x).data_ptr() % 16 == 4
+    y = rms_norm(x.view(T, H), w, 1e-6)
+    assert torch.equal(y, rms_norm(odd(x).view(T, H), odd(w), 1e-6))
+    assert torch.equal(rms_norm(x.view(T, H), None, 1e-6), rms_norm(odd(x).view(T, H), None, 1e-6))
+    a = gemma4_moe_inputs(x.view(T, H), w, w2, 1e-6)
+    b = gemma4_moe_inputs(odd(x).view(T, H), odd(w), odd(w2), 1e-6)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and torch.equal(a[0], y)
