@@ -284,7 +284,7 @@ def run_leg(args, pool: LayerPool, workload: str, headline: bool) -> dict:
     ops_dn = 2.0 * R * H * F
     layer_ops = ops_gu + ops_dn
     # the library's default switch to the f16-MFMA GEMMs: the rows that an expert averages (with copies)
-    mfma_path = T >= 128 and T * K >= (26 if spec.wtype == TYPE_Q4_0 else 30) * E
+    mfma_path = T >= 128 and T * K >= (22 if spec.wtype == TYPE_Q4_0 else 28) * E
 
     log(f"warmup {warmup} steps")
     for i in range(warmup):

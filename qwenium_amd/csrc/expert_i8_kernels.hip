@@ -37,24 +37,32 @@ typedef uint32_t u32x2i __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
 typedef const __attribute__((address_space(1))) u32x4a4* GlobalUnit;
 
-// 64-value block pairs per chunk: 288 (Q4_0) or 272 (Q8_0) consecutive bytes of a weight row
-template <int WT> constexpr int kI8Pairs = WT == kTypeQ4_0 ? 8 : 4;
-// a workgroup of at most ROWS (16 or 32) rows of one expert: a chunk's activation
-// quants [pair][lane group][slot][16 bytes] and block scales [block][slot], padded so
-// that neither the staging writes nor the operand reads meet in a bank
+// 64-value block pairs per chunk: 8 are 288 (Q4_0), 4 are 272 (Q8_0) consecutive
+// bytes of a weight row.  The Q4_0 gate/up of 32 rows takes 4 (144 bytes): it is bound
+// by its f64 steps, not by the stream, and three workgroups per CU hide more of them
+// (prompt of 1000 tokens, 35B-A3B shape: 200 -> 187 us; the down GEMM, whose rows are
+// one 8-pair chunk, lost: 91 -> 103).
+constexpr int i8_pairs(int wt, bool gateup, int rows) { return wt == kTypeQ4_0 && !(gateup && rows == 32) ? 8 : 4; }
+// workgroups per CU: three where the registers of 16 rows, or of the short chunks, allow it
+constexpr int i8_waves_per_simd(int wt, bool gateup, int rows) {
+    return rows == 16 || (wt == kTypeQ4_0 && gateup) ? 3 : 2;
+}
+
+// a workgroup of at most ROWS (16 or 32) rows of one expert, chunks of P pairs: a chunk's
+// activation quants [pair][lane group][slot][16 bytes] and block scales [block][slot], padded
+// so that neither the staging writes nor the operand reads meet in a bank
 template <int ROWS> constexpr int kI8APair = 4 * ROWS * 16 + 16;
 template <int ROWS> constexpr int kI8DBlock = ROWS + 4;
-template <int WT, int ROWS> constexpr int kI8ABytes = kI8Pairs<WT> * kI8APair<ROWS>;
-template <int WT, int ROWS> constexpr int kI8DBytes = 2 * kI8Pairs<WT> * kI8DBlock<ROWS> * 4;
+template <int P, int ROWS> constexpr int kI8ABytes = P * kI8APair<ROWS>;
+template <int P, int ROWS> constexpr int kI8DBytes = 2 * P * kI8DBlock<ROWS> * 4;
 
 template <int WT> constexpr int kI8PairBytes = 2 * BlockTraits<WT>::kBytes;
-template <int WT> constexpr int kI8RowBytes = kI8Pairs<WT> * kI8PairBytes<WT>;  // of a chunk: 288 or 272
-template <int WT> constexpr int kI8Units = kI8RowBytes<WT> / 16;                // 16-byte units per row: 18 or 17
-template <int WT> constexpr int kI8Ld = kI8RowBytes<WT> + (WT == kTypeQ4_0 ? 16 : 0);  // LDS row stride: 76 or 68 dwords
-template <int WT> constexpr int kI8WBytes = 32 * kI8Ld<WT>;                     // a wave's weight slab: 32 columns
-template <int WT, int ROWS>
-constexpr size_t kI8LdsBytes = 4 * (size_t)kI8WBytes<WT> + kI8ABytes<WT, ROWS> + kI8DBytes<WT, ROWS> + 2 * 4 * ROWS * 4;
-template <int ROWS> constexpr int kI8WavesPerSimd = ROWS == 16 ? 3 : 2;
+template <int WT, int P> constexpr int kI8RowBytes = P * kI8PairBytes<WT>;  // of a chunk
+// LDS row stride: 36, 76 or 68 dwords (columns 16 apart in four banks each way)
+template <int WT, int P> constexpr int kI8Ld = kI8RowBytes<WT, P> + (kI8RowBytes<WT, P> == 288 ? 16 : 0);
+template <int WT, int P> constexpr int kI8WBytes = 32 * kI8Ld<WT, P>;       // a wave's weight slab: 32 columns
+template <int WT, int P, int ROWS>
+constexpr size_t kI8LdsBytes = 4 * (size_t)kI8WBytes<WT, P> + kI8ABytes<P, ROWS> + kI8DBytes<P, ROWS> + 2 * 4 * ROWS * 4;
 
 struct I8Args {
     int H, F, E;
@@ -114,13 +122,13 @@ template <int J> struct I8Block<kTypeQ8_0, J> {
 
 // TAIL: the reduction length is not a multiple of a chunk, so a row's last chunk holds fewer pairs
 template <int WT, bool GATEUP, int ROWS, bool TAIL>
-__global__ __launch_bounds__(256, kI8WavesPerSimd<ROWS>) void k_expert_i8(I8Args a) {
+__global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_expert_i8(I8Args a) {
     extern __shared__ __align__(16) uint8_t s_dyn[];
-    constexpr int kPairs = kI8Pairs<WT>;
-    constexpr int kLd = kI8Ld<WT>;
-    uint8_t* s_a = s_dyn + 4 * kI8WBytes<WT>;
-    float* s_d = (float*)(s_a + kI8ABytes<WT, ROWS>);
-    float* s_amax = (float*)(s_a + kI8ABytes<WT, ROWS> + kI8DBytes<WT, ROWS>);  // [4 waves][ROWS]
+    constexpr int kPairs = i8_pairs(WT, GATEUP, ROWS);
+    constexpr int kLd = kI8Ld<WT, kPairs>;
+    uint8_t* s_a = s_dyn + 4 * kI8WBytes<WT, kPairs>;
+    float* s_d = (float*)(s_a + kI8ABytes<kPairs, ROWS>);
+    float* s_amax = (float*)(s_a + kI8ABytes<kPairs, ROWS> + kI8DBytes<kPairs, ROWS>);  // [4 waves][ROWS]
     int* s_sum = (int*)(s_amax + 4 * ROWS);
     // XCD-aware mapping (as the f16 GEMMs): XCD x takes every eighth tile, all column
     // groups of each; the shared expert's tiles, the fullest, come first.  The list
@@ -154,9 +162,9 @@ __global__ __launch_bounds__(256, kI8WavesPerSimd<ROWS>) void k_expert_i8(I8Args
     // The wave's slab of a chunk is 32 kU units of 16 bytes: unit s = 64 i + lane is
     // bytes 16 (s % kU) .. of column s / kU's chunk (columns 16 .. from wb1); kL
     // loads per lane, the spare lanes of the last repeat the last unit
-    constexpr int kU = kI8Units<WT>;
+    constexpr int kU = kI8RowBytes<WT, kPairs> / 16;
     constexpr int kL = (32 * kU + 63) / 64;
-    uint8_t* s_w = s_dyn + wave * kI8WBytes<WT>;
+    uint8_t* s_w = s_dyn + wave * kI8WBytes<WT, kPairs>;
     u32x4 wreg[kL];
     uint32_t woff[kL];
 #pragma unroll
@@ -180,7 +188,7 @@ __global__ __launch_bounds__(256, kI8WavesPerSimd<ROWS>) void k_expert_i8(I8Args
     // a uniform base made opaque: loads with a scalar base and one 32-bit offset per
     // lane, not a 64-bit running pointer per load
     auto base = [&](const uint8_t* w, int c) -> GlobalBytes {
-        const uint64_t b = (uint64_t)(uintptr_t)w + (uint64_t)(c * kI8RowBytes<WT>);
+        const uint64_t b = (uint64_t)(uintptr_t)w + (uint64_t)(c * kI8RowBytes<WT, kPairs>);
         return (GlobalBytes)(uintptr_t)(
             ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
             (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b));
@@ -400,8 +408,9 @@ __global__ __launch_bounds__(256, kI8WavesPerSimd<ROWS>) void k_expert_i8(I8Args
         case 2: run(std::integral_constant<int, 2>{}); break;
         case 3: run(std::integral_constant<int, 3>{}); break;
         case 4: run(std::integral_constant<int, 4>{}); break;
-        case 5:
+        case 5: if constexpr (ROWS > 16) run(std::integral_constant<int, 5>{}); break;
         case 6: if constexpr (ROWS > 16) run(std::integral_constant<int, 6>{}); break;
+        case 7: if constexpr (ROWS > 16) run(std::integral_constant<int, 7>{}); break;
         default: if constexpr (ROWS > 16) run(std::integral_constant<int, 8>{}); break;
     }
 }
@@ -430,9 +439,10 @@ int i8_tile_rows(const LayerDesc& L, int T) {
 template <int WT, bool GATEUP, int ROWS>
 static hipError_t launch_i8_rows(const LayerDesc& L, const Workspace& ws, int T, I8Args a, hipStream_t stream,
                                  hipEvent_t ev_start, hipEvent_t ev_stop) {
-    const bool tail = (a.K >> 6) % kI8Pairs<WT> != 0;
+    constexpr int kPairs = i8_pairs(WT, GATEUP, ROWS);
+    const bool tail = (a.K >> 6) % kPairs != 0;
     const auto kern = tail ? k_expert_i8<WT, GATEUP, ROWS, true> : k_expert_i8<WT, GATEUP, ROWS, false>;
-    constexpr size_t lds = kI8LdsBytes<WT, ROWS>;
+    constexpr size_t lds = kI8LdsBytes<WT, kPairs, ROWS>;
     // above the 64 KiB default dynamic LDS window: raise it (idempotent)
     const hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return err;

@@ -357,20 +357,20 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
         d.n_cu = n_cu;
     // token count from which the grouped f16-MFMA GEMMs (f32 sums, 128-row tiles)
     // replace the exact int8 ones: by the rows that an expert averages (T * top_k /
-    // n_experts), 40 (Q4_0) or 56 (Q8_0) over the GGUF rows, 26 or 30 with the
-    // chunk-major copies.  Layer us, int8 / f16: 35B-A3B Q4_0 328 / 375 at 31 rows,
-    // 423 / 408 at 44, with copies 256 / 292 at 22 and 328 / 311 at 31; Q8_0 490 /
-    // 554 at 44, 606 / 590 at 62, with copies 305 / 360 at 22 and 384 / 377 at 31;
-    // Gemma 4 292 / 343 at 28, 397 / 392 at 44, with copies 240 / 273 at 19 and 292
-    // / 284 at 28.
+    // n_experts), 36 (Q4_0) or 56 (Q8_0) over the GGUF rows, 22 or 28 with the
+    // chunk-major copies.  Layer us, int8 / f16: 35B-A3B Q4_0 332 / 358 at 31 rows,
+    // 388 / 385 at 37, with copies 245 / 262 at 19 and 332 / 293 at 31; Q8_0 504 /
+    // 537 at 47, with copies 326 / 339 at 25 and 385 / 360 at 31; Gemma 4 Q4_0 293 /
+    // 328 at 28, 360 / 346 at 37, with copies 219 / 230 at 16 and 255 / 243 at 22;
+    // Q8_0 526 / 549 at 62, 613 / 582 at 75, with copies 321 / 325 at 28.
     {
         const bool q4 = d.gu_type == QMOE_TYPE_Q4_0;
         auto from = [&](int rows) {
             const int64_t t = ((int64_t)rows * d.E + d.K - 1) / d.K;
             return (int)std::max<int64_t>(128, std::min<int64_t>(1 << 20, (t + 15) / 16 * 16));
         };
-        d.mfma_min_tokens = from(q4 ? 40 : 56);
-        d.mfma_min_tokens_pk = from(q4 ? 26 : 30);
+        d.mfma_min_tokens = from(q4 ? 36 : 56);
+        d.mfma_min_tokens_pk = from(q4 ? 22 : 28);
     }
     // token count from which routing runs the batched bf16-MFMA router: its cost is
     // nearly flat in T (its tiles split over more workgroups at small T), the exact
