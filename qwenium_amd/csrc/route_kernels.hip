@@ -16,8 +16,8 @@ namespace qmoe {
 // ---------------------------------------------------------------------------
 // R1: exact router logits of every token, for the debug copy when the batched
 // router runs (its own logits are approximate); the forward paths compute
-// theirs in k_route_decode (up to the batched router's threshold) or refine
-// the batched router's candidates in k_topk
+// theirs in k_route_decode (up to 16 tokens) and k_router_group (up to the batched
+// router's threshold) or refine the batched router's candidates in k_topk
 // ---------------------------------------------------------------------------
 struct RouterArgs {
     const float* x;         // [T][H] router input
@@ -547,8 +547,7 @@ struct TopkArgs {
     float norm_eps;
     float* x_scale;       // [T] the rows' RMSNorm scales (router block 0 writes them for the table launch)
     const double* x_ssq;  // [T][ssq_parts(H)] x's RMSNorm partial sums, or null (the router sums x itself)
-    int quant_rows;       // router launch over token groups: its blocks also write x's Q8_0 ...
-    int8_t* xq_qs;        // ... quants [T][H]
+    int8_t* xq_qs;        // group router: x's Q8_0 quants [T][H]
     float2* xq_ds;        // ... and {d, sum} [T][H/32]
     int32_t* topk_idx;    // [T][K]
     float* topk_w;        // [T][K]
@@ -1382,28 +1381,15 @@ __device__ __forceinline__ void shared_gateup_block(const TopkArgs& a, const Sha
 // tokens' scales (the tree over the chunks; the same bits in every block and in
 // the standalone RMSNorm).  Block 0 stores them for the table launch's Q8_0 of
 // x; the router input is (x * scale) * norm_w.
-template <int NSW, bool NORM, int RR = kRdRows>  // NSW: router slabs per wave (ceil(H/256/4)); RR: rows per block
-__global__ __launch_bounds__(1024) void k_route_decode(TopkArgs a0, float* logits0) {
+template <int NSW, bool NORM>  // NSW: router slabs per wave (ceil(H/256/4))
+__global__ __launch_bounds__(1024) void k_route_decode(TopkArgs a, float* logits) {
 #pragma clang fp contract(off)
-    constexpr int RVALS = RR * kRdTokSlots;  // (row, token) sums per wave
+    constexpr int RR = kRdRows, RVALS = RR * kRdTokSlots;  // (row, token) sums per wave
     __shared__ double s_part[RR][kRdParts][kTopkTokensPerBlock];
     __shared__ double s_chunk[NORM ? kTopkTokensPerBlock : 1][8];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     static_assert(!NORM || NSW <= 2, "the fused norm takes rows of at most 8 slabs");
-    // more than 16 tokens run in groups of 16: workgroup b takes router rows of
-    // block b % nbr for the tokens of group b / nbr; with quant_rows, router block
-    // rb of a group also writes the Q8_0 rows of its tokens rb + nbr * w (at the end)
-    const int nbr = (a0.E + a0.S + RR - 1) / RR;
-    const int gi = (int)blockIdx.x / nbr, rb = (int)blockIdx.x - gi * nbr;
-    const int tb = gi * kTopkTokensPerBlock;
-    if (a0.quant_rows && blockIdx.x == 0)  // the per-expert totals that the top-k blocks add into
-        for (int i = tid; i < kTotalCopies * a0.E; i += 1024) a0.hist[(uint64_t)a0.nblk * a0.E + i] = 0;
-    TopkArgs a = a0;  // this group's tokens
-    a.T = min(kTopkTokensPerBlock, a0.T - tb);
-    a.x = a0.x + (uint64_t)tb * a0.H;
-    a.x_scale = a0.x_scale + tb;
-    if (a0.x_ssq) a.x_ssq = a0.x_ssq + (uint64_t)tb * ssq_parts(a0.H);
-    float* logits = logits0 + (uint64_t)tb * (a0.E + 1);
+    const int rb = (int)blockIdx.x;
     const int E1 = a.E + a.S;
     const int nslab = a.H / kRdSlab;
     const int part = wave % kRdParts;
@@ -1562,9 +1548,73 @@ __global__ __launch_bounds__(1024) void k_route_decode(TopkArgs a0, float* logit
             for (int i = 0; i < kRdTokSlots; ++i)
                 if (kRdGroups * i + grp < a.T) a.x_scale[kRdGroups * i + grp] = xs[i];
     }
-    if (a0.quant_rows) {  // wave w: the group's token rb + nbr * w (at most one per block when nbr >= 16)
-        const int t = rb + nbr * wave;
-        if (t < a.T) quant_token_row(a0.xe, a0.H, tb + t, lane, a0.xq_qs, a0.xq_ds);
+}
+
+// The router from 17 tokens to the batched router's threshold: one workgroup per 16
+// tokens x 16 experts (the shared gate the last column), logits from
+// v_mfma_f64_16x16x4_f64 on the f32 operands widened, so each product is exact and
+// the sum is f64 as everywhere.  A matrix instruction does 16 vector FMAs' work in
+// half their time, needs one conversion per lane and operand, and leaves whole sums
+// per lane; the 16 waves take H / 16 columns each and meet in LDS once.  (Five rows
+// per workgroup on vector FMAs, each x value widened for five rows only and each sum
+// reduced over 64 lanes, took 30.4 us at 211 tokens of the 35B-A3B shape in three
+// rounds of workgroups, 13.2 at 64; this one takes 10.9 and 10.4, bound by the latency
+// of its loads.)  The first workgroups of the launch write x's
+// Q8_0, one wave per token.
+constexpr int kRgTile = 16;
+constexpr int kRgSteps = 8;  // 16-column steps with loads in flight per wave
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(1024) void k_router_group(TopkArgs a, float* logits) {
+    __shared__ double s_part[16][kRgTile * kRgTile];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int nq = (a.T + 15) / 16;
+    if ((int)blockIdx.x < nq) {
+        if (blockIdx.x == 0)  // the per-expert totals that the top-k blocks add into
+            for (int i = tid; i < kTotalCopies * a.E; i += 1024) a.hist[(uint64_t)a.nblk * a.E + i] = 0;
+        const int t = (int)blockIdx.x * 16 + wave;
+        if (t < a.T) quant_token_row(a.xe, a.H, t, lane, a.xq_qs, a.xq_ds);
+        return;
+    }
+    const int E1 = a.E + a.S, net = (E1 + kRgTile - 1) / kRgTile;
+    const int b = (int)blockIdx.x - nq;
+    const int t0 = (b / net) * kRgTile, e0 = (b % net) * kRgTile;
+    // A: token row lane % 16, B: router row lane % 16 (rows past the end repeat the last);
+    // lane group g = lane / 16 takes columns 4g .. 4g + 3 of each 16-column step, one MFMA per column
+    const int r = lane & 15, g = lane >> 4;
+    const int e = min(e0 + r, E1 - 1);
+    const float* xr = a.x + (uint64_t)min(t0 + r, a.T - 1) * a.H;
+    const float* wr = e < a.E ? a.w_router + (uint64_t)e * a.router_ld : a.w_sh_norm;
+    const int ns = a.H / 256;  // steps per wave
+    const int c0 = wave * 16 * ns + 4 * g;
+    f64x4 acc0 = {}, acc1 = {};
+    for (int s0 = 0; s0 < ns; s0 += kRgSteps) {
+        f32x4 xv[kRgSteps], wv[kRgSteps];
+#pragma unroll
+        for (int k = 0; k < kRgSteps; ++k) {
+            const int c = c0 + 16 * min(s0 + k, ns - 1);
+            xv[k] = *(const f32x4*)(xr + c);
+            wv[k] = *(const f32x4*)(wr + c);
+        }
+#pragma unroll
+        for (int k = 0; k < kRgSteps; ++k) {
+            if (s0 + k >= ns) break;  // uniform
+            acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[k].x, (double)wv[k].x, acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[k].y, (double)wv[k].y, acc1, 0, 0, 0);
+            acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[k].z, (double)wv[k].z, acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[k].w, (double)wv[k].w, acc1, 0, 0, 0);
+        }
+    }
+    // result i of a lane: token 4 i + g, router row lane % 16
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_part[wave][(4 * i + g) * kRgTile + r] = acc0[i] + acc1[i];
+    __syncthreads();
+    if (tid < kRgTile * kRgTile) {
+        double sum = s_part[0][tid];
+#pragma unroll
+        for (int w = 1; w < 16; ++w) sum = sum + s_part[w][tid];
+        const int t = t0 + tid / kRgTile, er = e0 + tid % kRgTile;
+        if (t < a.T && er < E1) logits[(uint64_t)t * (a.E + 1) + er] = (float)sum;
     }
 }
 
@@ -1762,19 +1812,6 @@ static const void* route_decode_kernel(int nsw, bool norm) {
         default: return nullptr;
     }
 }
-// The router over groups of 16 tokens: five rows per block for rows of at most
-// 2048 columns (a 256-expert layer's 52 blocks per group fill the CUs in one
-// round up to 64 tokens), two for wider rows (five would spill registers).
-static const void* route_group_kernel(int nsw, int* rows) {
-    *rows = nsw <= 2 ? 5 : kRdRows;
-    switch (nsw) {
-        case 1: return (const void*)k_route_decode<1, false, 5>;
-        case 2: return (const void*)k_route_decode<2, false, 5>;
-        case 3: return (const void*)k_route_decode<3, false>;
-        case 4: return (const void*)k_route_decode<4, false>;
-        default: return nullptr;
-    }
-}
 template <int SLPR>
 static const void* route_tables_for(int swt) {
     return swt == 0 ? (const void*)k_route_decode_tables<0, SLPR>
@@ -1814,7 +1851,6 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
     TopkArgs ta;
     ta.norm_w = nullptr;
     ta.x_ssq = nullptr;
-    ta.quant_rows = 0;
     ta.xq_qs = ws.xq_qs;
     ta.xq_ds = ws.xq_ds;
     ta.norm_eps = eps;
@@ -1854,13 +1890,16 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
     // on its four SIMDs)
     ta.tpb = kTopkTokensPerBlock;
     ta.nblk = (T + ta.tpb - 1) / ta.tpb;
-    const bool merge = !route_uses_mfma(L, T) && !route_decode_fused(L, T) && ta.nblk * L.E <= kTopkMergeMax;
+    // (the debug copies of the approximate logits and their bounds run the router that makes them)
+    const bool batched = route_uses_mfma(L, T) || ((dbg.approx || dbg.bound) && T > kTopkTokensPerBlock &&
+                                                   T >= L.router_debug_min_tokens);
+    const bool merge = !batched && !route_decode_fused(L, T) && ta.nblk * L.E <= kTopkMergeMax;
     if (!merge && T > kTopkTokensPerBlock) {
         while (ta.tpb > kTopkMinTokensPerBlock && (T + ta.tpb - 1) / ta.tpb < L.n_cu) ta.tpb >>= 1;
         ta.nblk = (T + ta.tpb - 1) / ta.tpb;
     }
     hipError_t err;
-    if (route_uses_mfma(L, T)) {
+    if (batched) {
         RouterMfmaArgs ma;
         ma.x = xr;
         ma.xe = x;
@@ -1970,21 +2009,10 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
             return err;
         return hipGetLastError();
     } else {
-        // the decode router over groups of 16 tokens, x's Q8_0 on the same launch
-        // (after each block's logits); then the top-k
-        ta.quant_rows = 1;
-        const int ngr = (T + kTopkTokensPerBlock - 1) / kTopkTokensPerBlock;
-        const int nsw = (L.H / kRdSlab + kRdParts - 1) / kRdParts;
-        int rows = 0;
-        const void* kern = route_group_kernel(nsw, &rows);
-        if (!kern) return hipErrorInvalidValue;
-        const int nb = (L.E + L.S + rows - 1) / rows;
-        float* logits = ws.logits;
-        void* args[] = {&ta, &logits};
-        if ((err = hipLaunchKernel(kern, dim3(nb * ngr), dim3(64 * kTopkTokensPerBlock), args, 0, stream)) !=
-            hipSuccess)
-            return err;
-        ta.quant_rows = 0;
+        // the router over tiles of 16 tokens, x's Q8_0 on the same launch; then the top-k
+        const int ngr = (T + kRgTile - 1) / kRgTile, net = (L.E + L.S + kRgTile - 1) / kRgTile;
+        hipLaunchKernelGGL(k_router_group, dim3(ngr + ngr * net), dim3(1024), 0, stream, ta, ws.logits);
+        if ((err = hipGetLastError()) != hipSuccess) return err;
         if (merge) {
             // the last top-k block runs the expert scan and the scatter: no more launches
             return launch_topk(topk_kernel<false, true>(L.E), ta, ws.sync, stream);

@@ -957,3 +957,15 @@ def test_norm_rows_aligned_equals_general(gpu, H):
     a = gemma4_moe_inputs(x.view(T, H), w, w2, 1e-6)
     b = gemma4_moe_inputs(odd(x).view(T, H), odd(w), odd(w2), 1e-6)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and torch.equal(a[0], y)
+
+
+@pytest.mark.parametrize("hidden,experts,T", [(256, 1, 17), (256, 15, 31), (512, 16, 32), (2304, 17, 33), (4096, 40, 47),
+                                              (1024, 300, 65)])
+def test_group_router_tile_edges(gpu, hidden, experts, T):
+    """The f64-MFMA router (17 tokens to the batched router): tiles of 16 tokens x 16 router rows
+    with every kind of remainder (the shared gate as a row of its own past 16 or 32), one to
+    sixteen 16-column steps per wave, 9 among them (a second batch of loads with one step):
+    logits within one ulp of the oracle's correctly rounded ones, routing and outputs equal."""
+    spec = LayerSpec(hidden, experts, min(2, experts), 64, True, TYPE_Q8_0)
+    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=500 + T)
+    assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0)
