@@ -379,12 +379,6 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
     // 64 experts of 1536 165 / 169 at 600, 206 / 201 at 1000 (the crossings lie from 700
     // tokens, with the RMSNorm folded into the batched router's preparation, to 1200)
     d.big_router_min_tokens = 720;
-    // the debug copies of the batched router's logits and bounds: from 224 tokens at the
-    // 35B-A3B shape, 272 at Gemma 4's
-    {
-        const double t = 216.0 * std::sqrt(524288.0 / ((double)d.E * (double)d.H));
-        d.router_debug_min_tokens = (int)std::max(128.0, std::min(1024.0, std::ceil(t / 16.0) * 16.0));
-    }
     if (const char* env = std::getenv("QMOE_MFMA_MIN_TOKENS")) {
         const long v = std::strtol(env, nullptr, 10);
         if (v >= 1) d.mfma_min_tokens = d.mfma_min_tokens_pk = (int)std::min<long>(v, 1 << 30);
@@ -397,7 +391,7 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
     // token count from which routing runs the batched bf16-MFMA router
     if (const char* env = std::getenv("QMOE_BIG_ROUTER_MIN_TOKENS")) {
         const long v = std::strtol(env, nullptr, 10);
-        if (v >= 1) d.big_router_min_tokens = d.router_debug_min_tokens = (int)std::min<long>(v, 1 << 30);
+        if (v >= 1) d.big_router_min_tokens = (int)std::min<long>(v, 1 << 30);
     }
     L->Hu = d.H;
     L->Fu = d.F;

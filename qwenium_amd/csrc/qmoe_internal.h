@@ -55,7 +55,6 @@ struct LayerDesc {
     int mfma_min_tokens = 128;              // token count from which the f16-MFMA GEMMs run over the GGUF rows
     int mfma_min_tokens_pk = 128;           // ... and with chunk-major copies (both set per shape)
     int big_router_min_tokens = 720;        // token count from which the bf16-MFMA router runs
-    int router_debug_min_tokens = 256;      // ... when the debug copies of its logits are asked for (set per shape)
     int dc_ahead = 2;                       // decode down+combine: steps with loads in flight (2 or 4)
     unsigned long long* expert_counts = nullptr;  // optional device [E]: += each forward's per-expert dispatches
     int act = 0;                            // 0 SwiGLU (silu(g)*u), 1 GeGLU-tanh (gelu(g)*u, ggml's fp16 table)

@@ -1890,9 +1890,8 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
     // on its four SIMDs)
     ta.tpb = kTopkTokensPerBlock;
     ta.nblk = (T + ta.tpb - 1) / ta.tpb;
-    // (the debug copies of the approximate logits and their bounds run the router that makes them)
-    const bool batched = route_uses_mfma(L, T) || ((dbg.approx || dbg.bound) && T > kTopkTokensPerBlock &&
-                                                   T >= L.router_debug_min_tokens);
+    // (also where debug copies are asked for: they describe the router that an ordinary call runs)
+    const bool batched = route_uses_mfma(L, T);
     const bool merge = !batched && !route_decode_fused(L, T) && ta.nblk * L.E <= kTopkMergeMax;
     if (!merge && T > kTopkTokensPerBlock) {
         while (ta.tpb > kTopkMinTokensPerBlock && (T + ta.tpb - 1) / ta.tpb < L.n_cu) ta.tpb >>= 1;
