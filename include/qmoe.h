@@ -123,7 +123,9 @@ const char* qmoe_last_error(void);
  * zero-padded copies of the weights at those widths (made here, one more copy
  * of the weights, any byte strides accepted) and every forward pads its rows
  * into the workspace and writes back the caller's width; results are those of
- * the unpadded layer (zero columns add exact zeros). */
+ * the unpadded layer (zero columns add exact zeros).  When the rows of an
+ * expert's or the shared expert's matrix lie so far apart that it spans 4 GiB
+ * or more, the layer keeps packed copies of the weights. */
 int qmoe_layer_create(const qmoe_tensor* w_router,
                       const qmoe_tensor* w_exp_gate,
                       const qmoe_tensor* w_exp_up,

@@ -190,7 +190,8 @@ size_t workspace_bytes(int T, int H, int E, int K, int F, Workspace* w, void* ba
 struct qmoe_layer {
     LayerDesc d;
     int Hu = 0, Fu = 0;         // the caller's widths; d.H, d.F are larger when the weights were padded
-    void* pad_base = nullptr;   // the padded weight copies (owned), or null
+    void* pad_base = nullptr;   // the padded or gathered weight copies (owned), or null
+    bool padded() const { return d.H != Hu || d.F != Fu; }
     int device = 0;
     qmoe_workspace* own_ws = nullptr;
     hipEvent_t phase_events[QMOE_N_PHASE_EVENTS] = {};
@@ -204,7 +205,28 @@ struct qmoe_workspace {
 
 namespace {
 
-// Zero-padded copies of the layer's weights at widths Hp >= H, Fp >= F (one
+// Rows of `width` bytes from one pitch to another on the device, one by one past
+// hipMemcpy2D's 31-bit pitch.
+hipError_t copy_rows(void* dst, uint64_t dst_pitch, const void* src, uint64_t src_pitch, uint64_t width, int rows) {
+    if (src_pitch < (1ull << 31)) return hipMemcpy2D(dst, dst_pitch, src, src_pitch, width, rows, hipMemcpyDeviceToDevice);
+    for (int r = 0; r < rows; ++r) {
+        const hipError_t err = hipMemcpy((uint8_t*)dst + r * dst_pitch, (const uint8_t*)src + r * src_pitch, width,
+                                         hipMemcpyDeviceToDevice);
+        if (err != hipSuccess) return err;
+    }
+    return hipSuccess;
+}
+
+// Whether a matrix of an expert spans 4 GiB or more: the expert GEMMs address its rows
+// with 32-bit byte offsets from the matrix's start.
+bool spans_4gib(const LayerDesc& d) {
+    const uint64_t gu = std::max(std::max(d.gate_nb1, d.up_nb1), std::max(d.sh_gate_nb1, d.sh_up_nb1));
+    const uint64_t dn = std::max(d.down_nb1, d.sh_down_nb1);
+    const uint64_t lim = 1ull << 32;
+    return gu > (lim - 1) / (uint64_t)d.F || dn > (lim - 1) / (uint64_t)d.H;
+}
+
+// Zero-padded, packed copies of the layer's weights at widths Hp >= H, Fp >= F (one
 // allocation, owned by the layer); the descriptor then points at them.
 hipError_t build_padded(qmoe_layer& L, int Hp, int Fp) {
     LayerDesc& d = L.d;
@@ -229,21 +251,20 @@ hipError_t build_padded(qmoe_layer& L, int Hp, int Fp) {
     uint8_t* sdown = p; p += n_sdn;
     float* snorm = (float*)p;
     err = hipMemset(base, 0, total);
-    const hipMemcpyKind k = hipMemcpyDeviceToDevice;
     if (err == hipSuccess)
-        err = hipMemcpy2D(router, (size_t)Hp * 4, d.w_router, (size_t)d.router_ld * 4, (size_t)H * 4, E, k);
+        err = copy_rows(router, (uint64_t)Hp * 4, d.w_router, d.router_ld * 4, (uint64_t)H * 4, E);
     const uint64_t wg = (uint64_t)(H / 32) * bg, wd = (uint64_t)(F / 32) * bd;  // real row bytes
     for (int e = 0; e < E && err == hipSuccess; ++e) {
-        err = hipMemcpy2D(gate + e * Fp * row_g, row_g, d.w_gate + e * d.gate_nb2, d.gate_nb1, wg, F, k);
-        if (err == hipSuccess) err = hipMemcpy2D(up + e * Fp * row_g, row_g, d.w_up + e * d.up_nb2, d.up_nb1, wg, F, k);
+        err = copy_rows(gate + e * Fp * row_g, row_g, d.w_gate + e * d.gate_nb2, d.gate_nb1, wg, F);
+        if (err == hipSuccess) err = copy_rows(up + e * Fp * row_g, row_g, d.w_up + e * d.up_nb2, d.up_nb1, wg, F);
         if (err == hipSuccess)
-            err = hipMemcpy2D(down + e * Hp * row_d, row_d, d.w_down + e * d.down_nb2, d.down_nb1, wd, H, k);
+            err = copy_rows(down + e * Hp * row_d, row_d, d.w_down + e * d.down_nb2, d.down_nb1, wd, H);
     }
     if (d.S && err == hipSuccess) {
-        err = hipMemcpy2D(sgate, row_g, d.w_sh_gate, d.sh_gate_nb1, wg, F, k);
-        if (err == hipSuccess) err = hipMemcpy2D(sup, row_g, d.w_sh_up, d.sh_up_nb1, wg, F, k);
-        if (err == hipSuccess) err = hipMemcpy2D(sdown, row_d, d.w_sh_down, d.sh_down_nb1, wd, H, k);
-        if (err == hipSuccess) err = hipMemcpy(snorm, d.w_sh_norm, (size_t)H * 4, k);
+        err = copy_rows(sgate, row_g, d.w_sh_gate, d.sh_gate_nb1, wg, F);
+        if (err == hipSuccess) err = copy_rows(sup, row_g, d.w_sh_up, d.sh_up_nb1, wg, F);
+        if (err == hipSuccess) err = copy_rows(sdown, row_d, d.w_sh_down, d.sh_down_nb1, wd, H);
+        if (err == hipSuccess) err = hipMemcpy(snorm, d.w_sh_norm, (size_t)H * 4, hipMemcpyDeviceToDevice);
     }
     if (err == hipSuccess) err = hipDeviceSynchronize();
     if (err != hipSuccess) {
@@ -395,10 +416,11 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
     }
     L->Hu = d.H;
     L->Fu = d.F;
-    if (d.H % 256 != 0 || d.F % 64 != 0) {
+    if (d.H % 256 != 0 || d.F % 64 != 0 || spans_4gib(d)) {
         // widths off the kernels' grid: zero-padded copies (n_embd to a multiple of
         // 256, ffn_dim of 64); the padded columns and rows meet zero weights and
-        // zero activations, so every real dot, sum and Q8_0 block keeps its value
+        // zero activations, so every real dot, sum and Q8_0 block keeps its value.
+        // Row strides beyond the GEMMs' 32-bit offsets: packed copies.
         const hipError_t err = build_padded(*L, (d.H + 255) / 256 * 256, (d.F + 63) / 64 * 64);
         if (err != hipSuccess) {
             delete L;
@@ -475,7 +497,7 @@ int qmoe_workspace_create(const qmoe_layer* like, int32_t max_tokens, qmoe_works
     const LayerDesc& d = like->d;
     qmoe_workspace* ws = new (std::nothrow) qmoe_workspace();
     if (!ws) return fail(QMOE_ERR_VALUE, "qmoe: host allocation failed");
-    const bool pad = like->pad_base != nullptr;
+    const bool pad = like->padded();
     const size_t bytes = qmoe::workspace_bytes(max_tokens, d.H, d.E, d.K, d.F, nullptr, nullptr, pad);
     void* base = nullptr;
     hipError_t err = hipMalloc(&base, bytes);
@@ -676,7 +698,7 @@ static int forward_impl(qmoe_layer* layer, qmoe_workspace* ws, const ForwardIn& 
                                         std::to_string(d.E) + "," + std::to_string(d.K) + "," + std::to_string(d.F) +
                                         "), got (" + std::to_string(w.H) + "," + std::to_string(w.E) + "," +
                                         std::to_string(w.K) + "," + std::to_string(w.F) + ")");
-    if (layer->pad_base && !in.padded_rows) return forward_padded(layer, ws, in, n_tokens, y, dbg, hip_stream);
+    if (layer->padded() && !in.padded_rows) return forward_padded(layer, ws, in, n_tokens, y, dbg, hip_stream);
     // buffers are sized for the workspace's (larger or equal) dims; kernels index with the layer's
     const Workspace& v = w;
     hipStream_t stream = (hipStream_t)hip_stream;
@@ -819,7 +841,7 @@ int qmoe_layer_forward_static(qmoe_layer* layer, const float* x, int32_t n_token
     if (n_tokens < 0) return fail(QMOE_ERR_VALUE, "qmoe: n_tokens expected >= 0, got " + std::to_string(n_tokens));
     if (n_tokens == 0) return QMOE_OK;
     const LayerDesc& d = layer->d;
-    const bool pad = layer->pad_base != nullptr;
+    const bool pad = layer->padded();
     const size_t need =
         kStaticSyncBytes + qmoe::workspace_bytes(n_tokens, d.H, d.E, d.K, d.F, nullptr, nullptr, pad);
     if (need > QMOE_STATIC_SCRATCH_BYTES)

@@ -910,18 +910,36 @@ def test_i8_experts_tile_edges(gpu, monkeypatch, wtype, hidden, ffn, experts, to
     assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0)
 
 
+class Strided(synthetic.GGMLTensor):
+    """Rows of a wider 2-d byte tensor."""
+
+    def desc(self):
+        d = super().desc()
+        d.nb[1] = self.data.shape[1]
+        d.nb[2] = d.nb[1] * self.ne[1]
+        return d
+
+
+def test_row_strides_beyond_32_bits(gpu):
+    """Gate rows 300 MB apart: 15 rows reach past 2^32 bytes.  Decode, the int8 GEMMs and the
+    f16 GEMMs give the packed layer's bits."""
+    spec = LayerSpec(256, 1, 1, 64, False, TYPE_Q4_0)
+    tensors = synthetic.make_layer_tensors(spec, 12)
+    rows = tensors["gate"].data.view(64, -1)
+    buf = torch.empty((64, 300_000_000), dtype=torch.uint8, device=rows.device)
+    buf[:, :rows.shape[1]] = rows
+    wide = dict(tensors, gate=Strided(buf, tensors["gate"].type, tensors["gate"].ne))
+    packed, strided = (synthetic.make_layer(spec, 12, tensors=t, prefill_copies=False) for t in (tensors, wide))
+    for T in (1, 17, 200):
+        x = synthetic.make_x(spec, T, 12)
+        assert torch.equal(packed.forward(x), strided.forward(x)), f"{T} tokens"
+    del wide, strided, buf
+    torch.cuda.empty_cache()
+
+
 def test_i8_experts_gate_up_strides(gpu):
     """Gate and up rows of different strides (views into wider rows): the int8 GEMM's two
     column bases; equal to the packed layer's results bit for bit."""
-    from qwenium_amd import GGMLTensor
-
-    class Strided(GGMLTensor):
-        def desc(self):
-            d = super().desc()
-            d.nb[1] = self.data.shape[1]
-            d.nb[2] = d.nb[1] * self.ne[1]
-            return d
-
     spec = LayerSpec(512, 8, 2, 128, False, TYPE_Q4_0)
     tensors = synthetic.make_layer_tensors(spec, 11)
     x = synthetic.make_x(spec, 50, 11)
