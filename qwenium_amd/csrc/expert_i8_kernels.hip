@@ -150,9 +150,9 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
 
     // this wave's 32 columns (two 16-column MFMA tiles): gate rows f0 .. f0 + 15 and
     // the same up rows, or down rows n0 .. n0 + 31.  Two waves share a Q8_0 block of h.
-    // A down workgroup runs n_cg consecutive column groups (128 columns each): its
-    // activations are staged once when one chunk holds them, and the next group's
-    // weights load while one is computed.
+    // A down workgroup runs n_cg consecutive column groups (128 columns each); more than
+    // one only where one chunk holds the activations: they are staged once, and the next
+    // group's weights load while one is computed.
     const int ncg = GATEUP ? 1 : min(a.n_cg, (a.H >> 7) - y * a.n_cg);
     const int f0 = y * 64 + 16 * wave, n0 = y * a.n_cg * 128 + 32 * wave;
     const uint32_t cs0 = (uint32_t)(sh ? a.sh0_nb1 : a.w0_nb1);
@@ -326,17 +326,18 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
 #pragma unroll
                 for (int i = 0; i < NQ; ++i) acc[ct][i] = 0.0;
             for (int c = 0; c < nchunk; ++c) {
-                const bool stage = nchunk > 1 || cg == 0;
+                const bool stage = cg == 0;
                 if (stage) {
-                    if (cg + c > 0) __syncthreads();  // the chunk before's activations are no longer read
+                    if (c > 0) __syncthreads();  // the chunk before's activations are no longer read
                     put_a();
                 }
                 put(c);  // (the wave's own slab)
                 if (stage) __syncthreads();
-                const bool wrap = c + 1 == nchunk;
-                if (!wrap || cg + 1 < ncg) {
-                    fetch(wrap ? cg + 1 : cg, wrap ? 0 : c + 1);
-                    if (nchunk > 1) fetch_a(wrap ? 0 : c + 1);
+                if (c + 1 < nchunk) {
+                    fetch(cg, c + 1);
+                    fetch_a(c + 1);
+                } else if (cg + 1 < ncg) {
+                    fetch(cg + 1, 0);
                 }
                 const int np = TAIL ? min(kPairs, npairs - kPairs * c) : kPairs;
 #pragma unroll 1
@@ -481,7 +482,18 @@ hipError_t launch_down_i8(const LayerDesc& L, const Workspace& ws, int T, hipStr
     a.sh0 = L.w_sh_down; a.sh0_nb1 = L.sh_down_nb1;
     a.a_qs = ws.hq_qs; a.a_ds = ws.hq_ds;
     a.K = L.F;
-    a.n_cg = 2;  // us at 211 tokens (35B-A3B Q4_0): 45.5 with 1, 43.7 with 2, 46.5 with 4, 54.2 with 8
+    // Two column groups per workgroup save the second staging of its rows where one chunk
+    // holds them and eight workgroups per CU are left (the kernel at 211 tokens, 35B-A3B Q4_0,
+    // us: 45.5 with 1, 43.7 with 2, 46.5 with 4, 54.2 with 8).  Elsewhere they only halve the
+    // grid.  Layer us, 2 / 1: 8 experts of ffn 4096, hidden 2048, 100 tokens 126.9 / 95.7; one
+    // expert of ffn 4096, 32 tokens 122.8 / 92.0; 16 experts of ffn 512, hidden 1024, 64 tokens
+    // 39.2 / 35.7; 35B-A3B Q8_0 (two chunks) at 100 tokens 193.5 / 185.6, Gemma 4 at 200 189.0 /
+    // 183.8; one chunk: 35B-A3B Q4_0 at 450 tokens 184.7 / 189.3, top-1 of 128 experts at 300
+    // 88.6 / 89.7 (2500 groups), top-4 of 32 at 100 61.9 / 60.6 (1000 groups).
+    const int rows = i8_tile_rows(L, T);
+    const bool one_chunk = (L.F >> 6) <= i8_pairs(L.dn_type, false, rows);
+    const int64_t groups = (int64_t)max_row_tiles(L, T, rows) * (L.H / 128);
+    a.n_cg = one_chunk && groups >= 8 * (int64_t)L.n_cu ? 2 : 1;
     a.n_y = (L.H / 128 + a.n_cg - 1) / a.n_cg;
     return L.dn_type == kTypeQ4_0 ? launch_i8<kTypeQ4_0, false>(L, ws, T, a, stream, nullptr, nullptr)
                                   : launch_i8<kTypeQ8_0, false>(L, ws, T, a, stream, nullptr, nullptr);
