@@ -70,7 +70,6 @@ constexpr int kSlotsPerRow = kLd / 8;       // sixteen-byte slots per row, the l
 constexpr int kASlots = kTM * kSlotsPerRow;
 constexpr int kAHalfs = kASlots * 8;
 constexpr int kDmaIters = (kASlots + 255) / 256;
-constexpr int kSinkBytes = 64 * 16;        // the last round's spare waves all land here
 static_assert(kASlots % 64 == 0, "a wave's staging slots are all real or all spare");
 constexpr int kScaleRounds = kTM * 4 / 256;  // scale dword slots per thread
 static_assert(kTM * 4 % 256 == 0, "scale slots");
@@ -85,7 +84,7 @@ constexpr int kHLd = 64 + 4;                // gate/up epilogue: g and u rows in
 constexpr int kOffSlots = kDmaIters + kScaleRounds;
 template <int WT> constexpr bool kOffLds = WT == kTypeQ8_0;
 template <int WT>
-constexpr size_t kF16LdsBytes = 2 * (size_t)kStageBytes + kSinkBytes + kTM * 8 + (kOffLds<WT> ? (size_t)kOffSlots * 256 * 4 : 0);
+constexpr size_t kF16LdsBytes = 2 * (size_t)kStageBytes + kTM * 8 + (kOffLds<WT> ? (size_t)kOffSlots * 256 * 4 : 0);
 static_assert(2 * 64 * kHLd * 4 <= 2 * (size_t)kStageBytes, "an epilogue pass's g and u rows fit the stage buffers");
 // Error model of the gate/up epilogue's f32 values.  The accumulation error of
 // g (n block terms summed by fma in f32) relative to max(|g|, rms of the
@@ -413,9 +412,9 @@ template <int WT, bool GATEUP, int ACT>
 __global__ __launch_bounds__(256, 3) void k_expert_f16(F16Args a) {
     extern __shared__ __align__(16) uint8_t s_dyn[];
     // [2 stages] {A quants [128][kLd] f16, block scale records [128][8] f16 (the
-    // 4 scales twice)}, the sink, A row offsets [128], scale row offsets [128]
+    // 4 scales twice)}, A row offsets [128], scale row offsets [128]
     uint8_t* s_stage = s_dyn;
-    uint32_t* s_rowoff = (uint32_t*)(s_dyn + 2 * kStageBytes + kSinkBytes);
+    uint32_t* s_rowoff = (uint32_t*)(s_dyn + 2 * kStageBytes);
     uint32_t* s_doff = s_rowoff + kTM;
     uint32_t* s_off = s_doff + kTM;  // kOffLds: [kOffSlots][256]
     // XCD-aware mapping (workgroups are dealt to the 8 XCDs round-robin): XCD x
@@ -470,9 +469,9 @@ __global__ __launch_bounds__(256, 3) void k_expert_f16(F16Args a) {
     const int nchunk = (nblk + 2 * kPPC - 1) / (2 * kPPC);
 
     // direct global->LDS staging of chunk c.  Quants: slot s = row * kSlotsPerRow
-    // + unit (the last unit is the row's padding); every wave issues exactly kDmaIters
-    // unconditional loads (a count the wait counters can track): slots past
-    // the buffer land in the sink, the padding unit reloads the chunk's first
+    // + unit (the last unit is the row's padding); a wave's 64 slots are loaded
+    // if one of them belongs to a row tile that has rows (every wait is for all
+    // loads, so their number is free), the padding unit reloads the chunk's first
     // 16 bytes of the row into a slot that is never read.  K is a multiple of
     // 64; with 128-wide chunks a last chunk holds 2 or 4 blocks, and a 2-block
     // one reads up to 128 bytes of quants and 4 bytes of scales past a row (the
@@ -507,9 +506,9 @@ __global__ __launch_bounds__(256, 3) void k_expert_f16(F16Args a) {
 #pragma unroll
         for (int it = 0; it < kDmaIters; ++it) {
             const int s0 = it * 256 + wave * 64;
-            if (s0 >= slots_nm) break;  // (wave-uniform)
-            const void* dst = s0 < kASlots ? (const void*)(st + s0 * 16) : (const void*)(s_stage + 2 * kStageBytes);
-            dma_lds16(a.a_q + k0, 2u * (kOffLds<WT> ? s_off[it * 256 + tid] : soff[it]), __builtin_amdgcn_readfirstlane(lds_addr(dst)));  // wave-uniform
+            if (s0 >= slots_nm) break;  // (wave-uniform; at most kASlots)
+            dma_lds16(a.a_q + k0, 2u * (kOffLds<WT> ? s_off[it * 256 + tid] : soff[it]),
+                      __builtin_amdgcn_readfirstlane(lds_addr(st + s0 * 16)));
         }
         // a 2-block last chunk: the odd dwords (blocks 2, 3, past the row) reload
         // blocks 0, 1, so every scale the MFMA multiplies (by 0 or not) is finite
@@ -867,9 +866,7 @@ template <int WT, bool GATEUP, int ACT>
 static hipError_t launch_f16(dim3 grid, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop, const F16Args& a) {
     const auto kern = k_expert_f16<WT, GATEUP, ACT>;
     constexpr size_t lds = kF16LdsBytes<WT>;
-    // above the 64 KiB default dynamic LDS window: raise it (idempotent)
-    hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (err != hipSuccess) return err;
+    static_assert(lds <= 64 * 1024, "within the default dynamic LDS window");
     launch_timed(kern, grid, dim3(256), lds, stream, ev_start, ev_stop, a);
     return hipGetLastError();
 }

@@ -444,9 +444,7 @@ static hipError_t launch_i8_rows(const LayerDesc& L, const Workspace& ws, int T,
     const bool tail = (a.K >> 6) % kPairs != 0;
     const auto kern = tail ? k_expert_i8<WT, GATEUP, ROWS, true> : k_expert_i8<WT, GATEUP, ROWS, false>;
     constexpr size_t lds = kI8LdsBytes<WT, kPairs, ROWS>;
-    // above the 64 KiB default dynamic LDS window: raise it (idempotent)
-    const hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (err != hipSuccess) return err;
+    static_assert(lds <= 64 * 1024, "within the default dynamic LDS window");
     a.max_tiles = max_row_tiles(L, T, ROWS);
     const dim3 grid((unsigned)(8 * ((a.max_tiles + 7) / 8) * a.n_y));
     launch_timed(kern, grid, dim3(256), lds, stream, ev_start, ev_stop, a);
