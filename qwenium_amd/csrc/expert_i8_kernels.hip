@@ -120,6 +120,15 @@ template <int J> struct I8Block<kTypeQ8_0, J> {
     __device__ __forceinline__ float scale() const { return fp16_to_f32(J == 0 ? d : d >> 16); }
 };
 
+// Orders this wave's LDS accesses before it with those after it, where lanes read what
+// others of the wave wrote and no barrier stands between (the hardware keeps a wave's LDS
+// operations in order: this keeps the compiler from moving them, and emits nothing).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // TAIL: the reduction length is not a multiple of a chunk, so a row's last chunk holds fewer pairs
 template <int WT, bool GATEUP, int ROWS, bool TAIL>
 __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_expert_i8(I8Args a) {
@@ -325,6 +334,7 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
             for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
                 for (int i = 0; i < NQ; ++i) acc[ct][i] = 0.0;
+            if (cg > 0) wave_lds_order();  // (the group before's reads of the slab)
             for (int c = 0; c < nchunk; ++c) {
                 const bool stage = cg == 0;
                 if (stage) {
@@ -333,6 +343,7 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
                 }
                 put(c);  // (the wave's own slab)
                 if (stage) __syncthreads();
+                else wave_lds_order();
                 if (c + 1 < nchunk) {
                     fetch(cg, c + 1);
                     fetch_a(c + 1);
