@@ -14,7 +14,7 @@
 // and chunk, 16 bytes per lane, into registers a chunk ahead (9.2 or 8.7 KB per
 // wave in flight, no padding rows, no chunk-major copy needed), and transposed to
 // the MFMA operand through the wave's own LDS slab, which no barrier orders; the
-// activations of a chunk, which the four waves share, take two.  144-byte pieces
+// activations of a chunk, which a part's waves share, take two.  144-byte pieces
 // of twice the columns ran at 3.6 instead of 4.2 TB/s.  The arithmetic is three
 // f64 instructions per output and block (convert, scale by dw, fma by dx), each at
 // an f32 instruction's rate on this chip, only for the groups of four rows that
@@ -42,10 +42,13 @@ typedef const __attribute__((address_space(1))) u32x4a4* GlobalUnit;
 // by its f64 steps, not by the stream, and three workgroups per CU hide more of them
 // (prompt of 1000 tokens, 35B-A3B shape: 200 -> 187 us; the down GEMM, whose rows are
 // one 8-pair chunk, lost: 91 -> 103).
-constexpr int i8_pairs(int wt, bool gateup, int rows) { return wt == kTypeQ4_0 && !(gateup && rows == 32) ? 8 : 4; }
+constexpr int i8_pairs(int wt, bool gateup, int rows, int ks = 1) {
+    return ks == 1 && wt == kTypeQ4_0 && !(gateup && rows == 32) ? 8 : 4;
+}
 // workgroups per CU: three where the registers of 16 rows, or of the short chunks, allow it
-constexpr int i8_waves_per_simd(int wt, bool gateup, int rows) {
-    return rows == 16 || (wt == kTypeQ4_0 && gateup) ? 3 : 2;
+// (a split workgroup is launched where the grid does not fill the CUs: two waves per SIMD)
+constexpr int i8_waves_per_simd(int wt, bool gateup, int rows, int ks) {
+    return ks == 1 && (rows == 16 || (wt == kTypeQ4_0 && gateup)) ? 3 : 2;
 }
 
 // a workgroup of at most ROWS (16 or 32) rows of one expert, chunks of P pairs: a chunk's
@@ -61,8 +64,10 @@ template <int WT, int P> constexpr int kI8RowBytes = P * kI8PairBytes<WT>;  // o
 // LDS row stride: 36, 76 or 68 dwords (columns 16 apart in four banks each way)
 template <int WT, int P> constexpr int kI8Ld = kI8RowBytes<WT, P> + (kI8RowBytes<WT, P> == 288 ? 16 : 0);
 template <int WT, int P> constexpr int kI8WBytes = 32 * kI8Ld<WT, P>;       // a wave's weight slab: 32 columns
-template <int WT, int P, int ROWS>
-constexpr size_t kI8LdsBytes = 4 * (size_t)kI8WBytes<WT, P> + kI8ABytes<P, ROWS> + kI8DBytes<P, ROWS> + 2 * 4 * ROWS * 4;
+template <int WT, int P, int ROWS, int CW>  // CW waves' weight slabs and their chunk's activations
+constexpr int kI8PartBytes = CW * kI8WBytes<WT, P> + kI8ABytes<P, ROWS> + kI8DBytes<P, ROWS>;
+template <int WT, int P, int ROWS, int CW, int KS>
+constexpr size_t kI8LdsBytes = KS * (size_t)kI8PartBytes<WT, P, ROWS, CW> + 2 * 4 * ROWS * 4;
 
 struct I8Args {
     int H, F, E;
@@ -129,15 +134,23 @@ __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
-// TAIL: the reduction length is not a multiple of a chunk, so a row's last chunk holds fewer pairs
-template <int WT, bool GATEUP, int ROWS, bool TAIL>
-__global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_expert_i8(I8Args a) {
+// TAIL: the reduction length is not a multiple of a chunk, so a row's last chunk holds fewer pairs.
+// KS: the workgroup's parts, each of CW waves (32 columns a wave) with slabs of its own; part p takes
+// chunks p, p + KS, ... of the reduction.  The parts' f64 sums, exact and so the same in any order,
+// meet in LDS before the epilogue.
+template <int WT, bool GATEUP, int ROWS, bool TAIL, int CW, int KS>
+__global__ __launch_bounds__(64 * CW * KS, i8_waves_per_simd(WT, GATEUP, ROWS, KS)) void k_expert_i8(I8Args a) {
     extern __shared__ __align__(16) uint8_t s_dyn[];
-    constexpr int kPairs = i8_pairs(WT, GATEUP, ROWS);
+    static_assert(KS == 1 || GATEUP, "the down GEMM is not split");
+    constexpr int kPairs = i8_pairs(WT, GATEUP, ROWS, KS);
     constexpr int kLd = kI8Ld<WT, kPairs>;
-    uint8_t* s_a = s_dyn + 4 * kI8WBytes<WT, kPairs>;
+    constexpr int kPart = kI8PartBytes<WT, kPairs, ROWS, CW>;
+    constexpr int kThreads = 64 * CW;  // of a part
+    const int part = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / kThreads);
+    uint8_t* s_part = s_dyn + part * kPart;
+    uint8_t* s_a = s_part + CW * kI8WBytes<WT, kPairs>;
     float* s_d = (float*)(s_a + kI8ABytes<kPairs, ROWS>);
-    float* s_amax = (float*)(s_a + kI8ABytes<kPairs, ROWS> + kI8DBytes<kPairs, ROWS>);  // [4 waves][ROWS]
+    float* s_amax = (float*)(s_dyn + KS * kPart);  // [CW waves][ROWS]
     int* s_sum = (int*)(s_amax + 4 * ROWS);
     // XCD-aware mapping (as the f16 GEMMs): XCD x takes every eighth tile, all column
     // groups of each; the shared expert's tiles, the fullest, come first.  The list
@@ -151,11 +164,12 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
     if (tile_id >= a.counters[1]) return;
     const int e = tile.x, p0 = tile.y, nr = tile.z;
     const bool sh = e >= a.E;
-    const int tid = threadIdx.x;
+    const int tid = KS == 1 ? threadIdx.x : threadIdx.x & (kThreads - 1);  // within the part
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int col = lane & 15, g = lane >> 4;
     const int npairs = a.K >> 6, nblk = a.K >> 5;
     const int nchunk = (npairs + kPairs - 1) / kPairs;
+    const int nstep = (nchunk + KS - 1) / KS;  // chunks per part; the last parts may have one fewer
 
     // this wave's 32 columns (two 16-column MFMA tiles): gate rows f0 .. f0 + 15 and
     // the same up rows, or down rows n0 .. n0 + 31.  Two waves share a Q8_0 block of h.
@@ -163,7 +177,7 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
     // one only where one chunk holds the activations: they are staged once, and the next
     // group's weights load while one is computed.
     const int ncg = GATEUP ? 1 : min(a.n_cg, (a.H >> 7) - y * a.n_cg);
-    const int f0 = y * 64 + 16 * wave, n0 = y * a.n_cg * 128 + 32 * wave;
+    const int f0 = y * 16 * CW + 16 * wave, n0 = y * a.n_cg * 128 + 32 * wave;
     const uint32_t cs0 = (uint32_t)(sh ? a.sh0_nb1 : a.w0_nb1);
     const uint32_t cs1 = GATEUP ? (uint32_t)(sh ? a.sh1_nb1 : a.w1_nb1) : cs0;
     const uint8_t* wb0 = (sh ? a.sh0 : a.w0 + (uint64_t)e * a.w0_nb2) + (uint64_t)(GATEUP ? f0 : n0) * cs0;
@@ -173,7 +187,7 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
     // loads per lane, the spare lanes of the last repeat the last unit
     constexpr int kU = kI8RowBytes<WT, kPairs> / 16;
     constexpr int kL = (32 * kU + 63) / 64;
-    uint8_t* s_w = s_dyn + wave * kI8WBytes<WT, kPairs>;
+    uint8_t* s_w = s_part + wave * kI8WBytes<WT, kPairs>;
     u32x4 wreg[kL];
     uint32_t woff[kL];
 #pragma unroll
@@ -231,11 +245,11 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
             }
         }
     };
-    fetch(0, 0);
+    if (KS == 1 || part < nchunk) fetch(0, part);
 
     // activations: thread t stages half-blocks of 16 values, half-block t % kHB of
-    // rows t / kHB, + 256 / kHB, ... of each chunk; even ones also the block's scale
-    constexpr int kHB = 4 * kPairs, kRS = 256 / kHB, kAR = ROWS / kRS;
+    // rows t / kHB, + kThreads / kHB, ... of each chunk; even ones also the block's scale
+    constexpr int kHB = 4 * kPairs, kRS = kThreads / kHB, kAR = ROWS / kRS;
     const int ahb = tid & (kHB - 1), ablk = ahb >> 1, ar0 = tid / kHB;
     uint32_t arow[kAR];
 #pragma unroll
@@ -275,7 +289,7 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
             if ((ahb & 1) == 0) s_d[ablk * kI8DBlock<ROWS> + slot] = WT == kTypeQ4_0 ? dreg[m] * 0.0625f : dreg[m];
         }
     };
-    fetch_a(0);
+    if (KS == 1 || part < nchunk) fetch_a(part);
 
     // the whole reduction and the epilogue for NQ groups of four rows
     auto run = [&](auto nq_c) {
@@ -335,22 +349,24 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
 #pragma unroll
                 for (int i = 0; i < NQ; ++i) acc[ct][i] = 0.0;
             if (cg > 0) wave_lds_order();  // (the group before's reads of the slab)
-            for (int c = 0; c < nchunk; ++c) {
+            for (int st = 0; st < nstep; ++st) {
+                const int c = part + KS * st;
+                const bool live = KS == 1 || c < nchunk;  // (uniform over the part)
                 const bool stage = cg == 0;
                 if (stage) {
-                    if (c > 0) __syncthreads();  // the chunk before's activations are no longer read
-                    put_a();
+                    if (st > 0) __syncthreads();  // the chunk before's activations are no longer read
+                    if (live) put_a();
                 }
-                put(c);  // (the wave's own slab)
+                if (live) put(c);  // (the wave's own slab)
                 if (stage) __syncthreads();
                 else wave_lds_order();
-                if (c + 1 < nchunk) {
-                    fetch(cg, c + 1);
-                    fetch_a(c + 1);
+                if (c + KS < nchunk) {
+                    fetch(cg, c + KS);
+                    fetch_a(c + KS);
                 } else if (cg + 1 < ncg) {
                     fetch(cg + 1, 0);
                 }
-                const int np = TAIL ? min(kPairs, npairs - kPairs * c) : kPairs;
+                const int np = !live ? 0 : TAIL ? min(kPairs, npairs - kPairs * c) : kPairs;
 #pragma unroll 1
                 for (int pp = 0; pp < np; ++pp) {
                     Ops o;
@@ -371,10 +387,29 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
             }
         }
         if (!GATEUP) return;
+        if constexpr (KS > 1) {
+            // over the slabs, which every wave is done with; part 0 then runs the epilogue
+            static_assert((KS - 1) * (ROWS / 4) * 2 * kThreads * 8 <= KS * kPart, "the sums fit");
+            double* red = (double*)s_dyn + tid;
+            __syncthreads();
+            if (part > 0)
+#pragma unroll
+                for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+                    for (int i = 0; i < NQ; ++i) red[kThreads * (2 * NQ * (part - 1) + NQ * ct + i)] = acc[ct][i];
+            __syncthreads();
+            if (part == 0)
+#pragma unroll
+                for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+                    for (int i = 0; i < NQ; ++i)
+#pragma unroll
+                        for (int p = 0; p < KS - 1; ++p) acc[ct][i] += red[kThreads * (2 * NQ * p + NQ * ct + i)];
+        }
         // h and its Q8_0, as swiglu_q8_block32: the 16 lanes of a group hold half of
         // a row's 32-value block, the other wave of the pair the other half; the
         // block's amax and quant sum meet in LDS
-        const int fb = y * 2 + (wave >> 1);
+        const int fb = y * (CW / 2) + (wave >> 1);
         float h[NQ];
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
@@ -384,7 +419,7 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
             amax = dpp8_max<kDppQuadXor2>(amax);
             amax = dpp8_max<kDppRowHalfMirror>(amax);
             amax = dpp8_max<kDppRowMirror>(amax);
-            if (col == 0) s_amax[wave * ROWS + 4 * i + g] = amax;
+            if (col == 0 && part == 0) s_amax[wave * ROWS + 4 * i + g] = amax;
         }
         __syncthreads();
         float d[NQ];
@@ -401,11 +436,11 @@ __global__ __launch_bounds__(256, i8_waves_per_simd(WT, GATEUP, ROWS)) void k_ex
             sum[i] = dpp8_add<kDppQuadXor2>(sum[i]);
             sum[i] = dpp8_add<kDppRowHalfMirror>(sum[i]);
             sum[i] = dpp8_add<kDppRowMirror>(sum[i]);
-            if ((wave & 1) && col == 0) s_sum[wave * ROWS + r] = sum[i];
-            if (r < nr) a.h_qs[(uint64_t)(p0 + r) * a.F + f0 + col] = (int8_t)q;
+            if ((wave & 1) && col == 0 && part == 0) s_sum[wave * ROWS + r] = sum[i];
+            if (r < nr && part == 0) a.h_qs[(uint64_t)(p0 + r) * a.F + f0 + col] = (int8_t)q;
         }
         __syncthreads();
-        if (!(wave & 1) && col == 0) {
+        if (!(wave & 1) && col == 0 && part == 0) {
 #pragma unroll
             for (int i = 0; i < NQ; ++i) {
                 const int r = 4 * i + g;
@@ -448,26 +483,61 @@ int i8_tile_rows(const LayerDesc& L, int T) {
     return (int64_t)T * L.K > 14 * (int64_t)L.E ? 32 : 16;
 }
 
-template <int WT, bool GATEUP, int ROWS>
-static hipError_t launch_i8_rows(const LayerDesc& L, const Workspace& ws, int T, I8Args a, hipStream_t stream,
-                                 hipEvent_t ev_start, hipEvent_t ev_stop) {
-    constexpr int kPairs = i8_pairs(WT, GATEUP, ROWS);
-    const bool tail = (a.K >> 6) % kPairs != 0;
-    const auto kern = tail ? k_expert_i8<WT, GATEUP, ROWS, true> : k_expert_i8<WT, GATEUP, ROWS, false>;
-    constexpr size_t lds = kI8LdsBytes<WT, kPairs, ROWS>;
-    static_assert(lds <= 64 * 1024, "within the default dynamic LDS window");
+template <int WT, bool GATEUP, int ROWS, bool TAIL, int CW, int KS>
+static hipError_t launch_i8_inst(const LayerDesc& L, int T, I8Args a, hipStream_t stream, hipEvent_t ev_start,
+                                 hipEvent_t ev_stop) {
+    const auto kern = k_expert_i8<WT, GATEUP, ROWS, TAIL, CW, KS>;
+    constexpr size_t lds = kI8LdsBytes<WT, i8_pairs(WT, GATEUP, ROWS, KS), ROWS, CW, KS>;
+    static_assert(lds <= 160 * 1024, "a CU's LDS");
+    if constexpr (lds > 64 * 1024) {  // above the default dynamic LDS window: raise it (idempotent)
+        const hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (err != hipSuccess) return err;
+    }
     a.max_tiles = max_row_tiles(L, T, ROWS);
     const dim3 grid((unsigned)(8 * ((a.max_tiles + 7) / 8) * a.n_y));
-    launch_timed(kern, grid, dim3(256), lds, stream, ev_start, ev_stop, a);
+    launch_timed(kern, grid, dim3(64 * CW * KS), lds, stream, ev_start, ev_stop, a);
     return hipGetLastError();
 }
 
+// A gate/up grid that leaves CUs idle (tiles go to the XCDs in turn: fewer than eight reach
+// as many XCDs only) is bound by what one CU can fetch: workgroups of 32 ffn columns, two waves
+// of them, each half of the reduction; below half the CUs four waves, each a quarter.  Layer us,
+// whole workgroups / halves / quarters: 16 experts of ffn 512, hidden 1024, Q8_0, 64 tokens (184
+// workgroups) 35.3 / 33.4 / 33.2; top-1 of 128 of ffn 512, hidden 2048, 17 tokens (152) 41.6 /
+// 36.6 / 38.3; 64 of ffn 64, hidden 4096, 17 tokens (70) 64.3 / 53.8 / 51.4; 16 of ffn 128, hidden
+// 4096, Q8_0, 13 tokens (32) 55.2 / 43.6 / 38.8; past the CUs' number level or slower (32 of ffn
+// 1024, hidden 4096, 64 tokens, 736 workgroups 101.4 / 104.9 / 116.7).
+static int i8_gateup_parts(const LayerDesc& L, int64_t tiles, int npairs) {
+    const int64_t wgs = tiles * (L.F / 64), cus = (int64_t)L.n_cu * std::min<int64_t>(tiles, 8) / 8;
+    if (2 * wgs <= cus && npairs >= 16) return 4;
+    return wgs <= cus && npairs >= 8 ? 2 : 1;
+}
+
+template <int WT, bool GATEUP, int ROWS>
+static hipError_t launch_i8_rows(const LayerDesc& L, int T, I8Args a, hipStream_t stream, hipEvent_t ev_start,
+                                 hipEvent_t ev_stop) {
+    const int npairs = a.K >> 6;
+    if constexpr (GATEUP) {
+        const int parts = i8_gateup_parts(L, max_row_tiles(L, T, ROWS), npairs);
+        if (parts > 1) {
+            a.n_y = L.F / 32;
+            return parts == 4 ? launch_i8_inst<WT, true, ROWS, false, 2, 4>(L, T, a, stream, ev_start, ev_stop)
+                              : launch_i8_inst<WT, true, ROWS, false, 2, 2>(L, T, a, stream, ev_start, ev_stop);
+        }
+    }
+    // (n_embd is a multiple of 256: the gate/up's chunks of four pairs are whole)
+    if constexpr (!GATEUP || i8_pairs(WT, GATEUP, ROWS) != 4)
+        if (npairs % i8_pairs(WT, GATEUP, ROWS) != 0)
+            return launch_i8_inst<WT, GATEUP, ROWS, true, 4, 1>(L, T, a, stream, ev_start, ev_stop);
+    return launch_i8_inst<WT, GATEUP, ROWS, false, 4, 1>(L, T, a, stream, ev_start, ev_stop);
+}
+
 template <int WT, bool GATEUP>
-static hipError_t launch_i8(const LayerDesc& L, const Workspace& ws, int T, const I8Args& a, hipStream_t stream,
-                            hipEvent_t ev_start, hipEvent_t ev_stop) {
+static hipError_t launch_i8(const LayerDesc& L, int T, const I8Args& a, hipStream_t stream, hipEvent_t ev_start,
+                            hipEvent_t ev_stop) {
     const bool wide = i8_tile_rows(L, T) == 32;
-    return wide ? launch_i8_rows<WT, GATEUP, 32>(L, ws, T, a, stream, ev_start, ev_stop)
-                : launch_i8_rows<WT, GATEUP, 16>(L, ws, T, a, stream, ev_start, ev_stop);
+    return wide ? launch_i8_rows<WT, GATEUP, 32>(L, T, a, stream, ev_start, ev_stop)
+                : launch_i8_rows<WT, GATEUP, 16>(L, T, a, stream, ev_start, ev_stop);
 }
 
 hipError_t launch_gateup_i8(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream, hipEvent_t ev_start,
@@ -481,8 +551,8 @@ hipError_t launch_gateup_i8(const LayerDesc& L, const Workspace& ws, int T, hipS
     a.K = L.H;
     a.n_y = L.F / 64;
     a.n_cg = 1;
-    return L.gu_type == kTypeQ4_0 ? launch_i8<kTypeQ4_0, true>(L, ws, T, a, stream, ev_start, ev_stop)
-                                  : launch_i8<kTypeQ8_0, true>(L, ws, T, a, stream, ev_start, ev_stop);
+    return L.gu_type == kTypeQ4_0 ? launch_i8<kTypeQ4_0, true>(L, T, a, stream, ev_start, ev_stop)
+                                  : launch_i8<kTypeQ8_0, true>(L, T, a, stream, ev_start, ev_stop);
 }
 
 hipError_t launch_down_i8(const LayerDesc& L, const Workspace& ws, int T, hipStream_t stream) {
@@ -504,8 +574,8 @@ hipError_t launch_down_i8(const LayerDesc& L, const Workspace& ws, int T, hipStr
     const int64_t groups = (int64_t)max_row_tiles(L, T, rows) * (L.H / 128);
     a.n_cg = one_chunk && groups >= 8 * (int64_t)L.n_cu ? 2 : 1;
     a.n_y = (L.H / 128 + a.n_cg - 1) / a.n_cg;
-    return L.dn_type == kTypeQ4_0 ? launch_i8<kTypeQ4_0, false>(L, ws, T, a, stream, nullptr, nullptr)
-                                  : launch_i8<kTypeQ8_0, false>(L, ws, T, a, stream, nullptr, nullptr);
+    return L.dn_type == kTypeQ4_0 ? launch_i8<kTypeQ4_0, false>(L, T, a, stream, nullptr, nullptr)
+                                  : launch_i8<kTypeQ8_0, false>(L, T, a, stream, nullptr, nullptr);
 }
 
 }  // namespace qmoe

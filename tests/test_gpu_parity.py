@@ -896,14 +896,18 @@ def test_python_checks_on_device_operands(gpu):
 @pytest.mark.parametrize("wtype", [TYPE_Q4_0, TYPE_Q8_0])
 @pytest.mark.parametrize("hidden,ffn", [(256, 64), (512, 192), (768, 704), (1280, 576)])
 @pytest.mark.parametrize("experts,top_k,T", [
-    (1, 1, 17), (1, 1, 31), (1, 1, 32), (1, 1, 33), (1, 1, 129),  # all rows on one expert: 32-row tiles and their remainders
-    (16, 2, 17), (16, 2, 40), (16, 2, 112), (16, 2, 113),         # 1 to ~20 rows: every group of four, both tile heights
+    # all rows on one expert: 32-row tiles whose last group of four rows is full or holds one row
+    (1, 1, 17), (1, 1, 20), (1, 1, 21), (1, 1, 24), (1, 1, 25), (1, 1, 28), (1, 1, 29), (1, 1, 31), (1, 1, 32),
+    (1, 1, 33), (1, 1, 129),
+    (16, 2, 17), (16, 2, 40), (16, 2, 112), (16, 2, 113),  # 1 to ~20 rows, both tile heights
+    (64, 4, 40), (64, 4, 300),                             # grids past the CUs at ffn 576 and 704
 ])
 def test_i8_experts_tile_edges(gpu, monkeypatch, wtype, hidden, ffn, experts, top_k, T):
-    """Tiles of 16 and 32 rows with every remainder, reduction lengths that end in a partial
-    chunk (Q4_0 chunks of 8 block pairs, Q8_0 of 4: 1 to 11 pairs here) and ffn widths of odd
-    column groups: routing bit-exact, h quants and outputs bit-identical to the oracle's (the
-    sums are exact in f64 on both sides)."""
+    """Tiles of 16 and 32 rows at both ends of every group of four, reduction lengths that end
+    in a partial chunk (Q4_0 chunks of 8 block pairs, Q8_0 of 4: 1 to 20 pairs here), ffn widths
+    of odd column groups, and gate/up workgroups that are whole or split in two or four parts
+    (of equal and unequal numbers of chunks): routing bit-exact, h quants and outputs
+    bit-identical to the oracle's (the sums are exact in f64 on both sides)."""
     monkeypatch.setenv("QMOE_MFMA_MIN_TOKENS", "100000")
     spec = LayerSpec(hidden, experts, top_k, ffn, True, wtype)
     y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=300 + T + hidden)
