@@ -1381,7 +1381,10 @@ __device__ __forceinline__ void shared_gateup_block(const TopkArgs& a, const Sha
 // tokens' scales (the tree over the chunks; the same bits in every block and in
 // the standalone RMSNorm).  Block 0 stores them for the table launch's Q8_0 of
 // x; the router input is (x * scale) * norm_w.
-template <int NSW, bool NORM>  // NSW: router slabs per wave (ceil(H/256/4))
+// GROUPS: more than 16 tokens in groups of 16: workgroup b takes the router rows of block
+// b % nbr for the tokens of group b / nbr, then writes the Q8_0 of the group's tokens
+// b % nbr + nbr * w.
+template <int NSW, bool NORM, bool GROUPS = false>  // NSW: router slabs per wave (ceil(H/256/4))
 __global__ __launch_bounds__(1024) void k_route_decode(TopkArgs a, float* logits) {
 #pragma clang fp contract(off)
     constexpr int RR = kRdRows, RVALS = RR * kRdTokSlots;  // (row, token) sums per wave
@@ -1389,7 +1392,17 @@ __global__ __launch_bounds__(1024) void k_route_decode(TopkArgs a, float* logits
     __shared__ double s_chunk[NORM ? kTopkTokensPerBlock : 1][8];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     static_assert(!NORM || NSW <= 2, "the fused norm takes rows of at most 8 slabs");
-    const int rb = (int)blockIdx.x;
+    static_assert(!NORM || !GROUPS, "the fused norm is decode's");
+    const int nbr = (a.E + a.S + RR - 1) / RR;
+    const int rb = GROUPS ? (int)blockIdx.x % nbr : (int)blockIdx.x;
+    const int tb = GROUPS ? (int)blockIdx.x / nbr * kTopkTokensPerBlock : 0;  // the group's first token
+    if constexpr (GROUPS) {
+        if (blockIdx.x == 0)  // the per-expert totals that the top-k blocks add into
+            for (int i = tid; i < kTotalCopies * a.E; i += 1024) a.hist[(uint64_t)a.nblk * a.E + i] = 0;
+        a.T = min(kTopkTokensPerBlock, a.T - tb);
+        a.x += (uint64_t)tb * a.H;
+        logits += (uint64_t)tb * (a.E + 1);
+    }
     const int E1 = a.E + a.S;
     const int nslab = a.H / kRdSlab;
     const int part = wave % kRdParts;
@@ -1547,6 +1560,10 @@ __global__ __launch_bounds__(1024) void k_route_decode(TopkArgs a, float* logits
 #pragma unroll
             for (int i = 0; i < kRdTokSlots; ++i)
                 if (kRdGroups * i + grp < a.T) a.x_scale[kRdGroups * i + grp] = xs[i];
+    }
+    if constexpr (GROUPS) {
+        const int t = rb + nbr * wave;
+        if (t < a.T) quant_token_row(a.xe, a.H, tb + t, lane, a.xq_qs, a.xq_ds);
     }
 }
 
@@ -1812,6 +1829,26 @@ static const void* route_decode_kernel(int nsw, bool norm) {
         default: return nullptr;
     }
 }
+// 17 tokens and more: the decode router's blocks of two rows over groups of 16 tokens (nbr x ngr
+// blocks) where they fill the CUs once at most; the f64-MFMA tiles are an eighth as many, each
+// bound by its own CU's f64 rate (6.8 us at 4096 columns).  Layer us, tiles / row pairs: 16
+// experts at 17 to 200 tokens 1.1 to 1.6 less at 1024 columns, 3 to 4 at 2048, 7 to 9 at 4096 (the
+// router 16.2 -> 8.6); 64 experts, 4096 columns, 100 tokens (231 blocks) 7.2 less, 200 (429) 1.1
+// less, 300 (627) 4.1 more; 128 experts, 2048 columns, 64 tokens (256) 3.8 less, 200 (832) 5.2
+// more.  512 columns are level, and below four blocks per group too few waves quantize x (one
+// expert 0.7 to 2 more).
+static bool router_in_row_pairs(const LayerDesc& L, int nbr, int ngr) {
+    return L.H >= 1024 && nbr >= 4 && nbr * ngr <= L.n_cu;
+}
+static const void* route_groups_kernel(int nsw) {
+    switch (nsw) {
+        case 1: return (const void*)k_route_decode<1, false, true>;
+        case 2: return (const void*)k_route_decode<2, false, true>;
+        case 3: return (const void*)k_route_decode<3, false, true>;
+        case 4: return (const void*)k_route_decode<4, false, true>;
+        default: return nullptr;
+    }
+}
 template <int SLPR>
 static const void* route_tables_for(int swt) {
     return swt == 0 ? (const void*)k_route_decode_tables<0, SLPR>
@@ -2010,7 +2047,17 @@ static hipError_t launch_route_tables(const LayerDesc& L, const Workspace& ws, c
     } else {
         // the router over tiles of 16 tokens, x's Q8_0 on the same launch; then the top-k
         const int ngr = (T + kRgTile - 1) / kRgTile, net = (L.E + L.S + kRgTile - 1) / kRgTile;
-        hipLaunchKernelGGL(k_router_group, dim3(ngr + ngr * net), dim3(1024), 0, stream, ta, ws.logits);
+        const int nbr = (L.E + L.S + kRdRows - 1) / kRdRows;
+        if (router_in_row_pairs(L, nbr, ngr)) {
+            const void* kern = route_groups_kernel((L.H / kRdSlab + kRdParts - 1) / kRdParts);
+            if (!kern) return hipErrorInvalidValue;
+            float* logits = ws.logits;
+            void* args[] = {&ta, &logits};
+            if ((err = hipLaunchKernel(kern, dim3(nbr * ngr), dim3(64 * kTopkTokensPerBlock), args, 0, stream)) != hipSuccess)
+                return err;
+        } else {
+            hipLaunchKernelGGL(k_router_group, dim3(ngr + ngr * net), dim3(1024), 0, stream, ta, ws.logits);
+        }
         if ((err = hipGetLastError()) != hipSuccess) return err;
         if (merge) {
             // the last top-k block runs the expert scan and the scatter: no more launches

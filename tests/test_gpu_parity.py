@@ -159,9 +159,8 @@ def test_decode_hidden_sizes(gpu, spec, T):
                                     (LayerSpec(3072, 96, 6, 512, True, TYPE_Q4_0), 40),
                                     (LayerSpec(1280, 40, 4, 512, False, TYPE_Q4_0), 50)])
 def test_grouped_router_hidden_sizes(gpu, spec, T):
-    """17 tokens to the batched router's threshold (the router over groups of 16 tokens, x's Q8_0 rows written by its
-    blocks) at hidden 4096 / 3072 (two router rows per block) and 1280 (five rows per
-    block, the last wave with one slab fewer, 9 blocks per group for 16 tokens)."""
+    """17 tokens to the batched router's threshold at hidden 4096 / 3072 / 1280: four, three and two
+    256-column slabs per router wave, x's Q8_0 rows written by the router's blocks."""
     y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=310 + T)
     assert_parity(y, got, y_ref, d_ref, spec)
 
@@ -992,3 +991,16 @@ def test_group_router_tile_edges(gpu, hidden, experts, T):
     spec = LayerSpec(hidden, experts, min(2, experts), 64, True, TYPE_Q8_0)
     y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=500 + T)
     assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0)
+
+
+@pytest.mark.parametrize("hidden,experts,T", [(1024, 7, 17), (1024, 8, 64), (2048, 31, 33), (2816, 6, 200), (3840, 30, 255),
+                                              (4096, 64, 112), (4096, 64, 113)])
+def test_row_pair_router_groups(gpu, hidden, experts, T):
+    """17 tokens and more where the router's blocks of two rows over groups of 16 tokens fit the
+    CUs once: one to four slabs per wave (fewer in the last waves), an odd last row, whole and
+    partial groups, the fewest blocks per group (four: each quantizes up to four tokens), and the
+    most blocks before the f64-MFMA tiles take over (33 x 7 against 33 x 8): logits within one
+    ulp of the oracle's, routing and outputs equal."""
+    spec = LayerSpec(hidden, experts, min(2, experts), 64, True, TYPE_Q8_0)
+    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=600 + T)
+    assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0, mfma=T * 2 >= 28 * experts and T >= 128)
