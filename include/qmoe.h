@@ -186,7 +186,7 @@ int qmoe_layer_forward(qmoe_layer* layer, qmoe_workspace* ws,
  * after each use) is zero when the library loads, and a first call on a
  * stream that is not being captured also clears it and waits for that clear
  * (the one synchronisation this entry point performs).  Sizes whose
- * scratch exceeds the maximum (at the 35B-A3B shape: above about 100 tokens)
+ * scratch exceeds the maximum (at the 35B-A3B shape: above 94 tokens)
  * fail with QMOE_ERR_CAPACITY.  Every call on one GPU shares that GPU's
  * array: calls that overlap in time on one GPU (other streams, other threads)
  * race and must not be issued; calls ordered on one stream are fine. */

@@ -156,11 +156,10 @@ size_t workspace_bytes(int T, int H, int E, int K, int F, Workspace* w, void* ba
     ws.counters = (int32_t*)take(qmoe::kCounters * sizeof(int32_t));
     ws.sync = (int32_t*)take(kSyncWords * sizeof(int32_t));
     ws.tiles = (int4*)take((size_t)max_tiles * sizeof(int4));
-    ws.gubuf = (float2*)take(R * F * sizeof(float2));
-    ws.h_q = (_Float16*)ws.gubuf;  // R*F*2 bytes of the R*F*8 (the rest is its padding)
     // built with 128-wide k chunks, the prefill GEMMs stage whole chunks: a
     // 64-wide last chunk reads up to 128 bytes of quants and 4 bytes of scales
     // past a row, so the four A buffers end in 256 bytes of padding
+    ws.h_q = (_Float16*)take(R * F * sizeof(_Float16) + 256);
     ws.h_d = (uint16_t*)take(R * (F / 32) * sizeof(uint16_t) + 256);
     ws.x_q = (_Float16*)take((size_t)T * H * sizeof(_Float16) + 256);
     ws.x_d = (uint16_t*)take((size_t)T * (H / 32) * sizeof(uint16_t) + 256);

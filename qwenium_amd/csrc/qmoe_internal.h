@@ -100,13 +100,12 @@ struct Workspace {
     int32_t* counters = nullptr;  // [kCounters]
     int32_t* sync = nullptr;      // [kSyncWords] zeroed at creation: the merged top-k's finished-workgroup counter
     int4* tiles = nullptr;        // [max tiles] {expert, row0, nrows, 0}
-    float2* gubuf = nullptr;      // [R][F] the room of h_q
     int8_t* hq_qs = nullptr;      // [R][F]   Q8_0 quants of h = silu(g)*u
     float2* hq_ds = nullptr;      // [R][F/32] {d, bitcast(sum q)}
     // prefill GEMM operands: Q8_0 quants as exact f16 values and fp16 block scales
     _Float16* x_q = nullptr;      // [T][H] x (the experts' input)
     uint16_t* x_d = nullptr;      // [T][H/32]
-    _Float16* h_q = nullptr;      // [R][F] h (in gubuf)
+    _Float16* h_q = nullptr;      // [R][F] h
     uint16_t* h_d = nullptr;      // [R][F/32]
     // batched router operands: bf16 hi/lo splits of the router input and weights, row norms
     uint16_t* rx_split = nullptr; // [2][T][H] (hi, lo)

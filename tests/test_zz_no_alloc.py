@@ -25,14 +25,16 @@ def test_static_forward_rejects_sizes_above_the_scratch():
         rc = L.qmoe_layer_forward_static(h, FAKE, 4096, FAKE, None, None)
         assert rc == QMOE_ERR_CAPACITY
         assert "static scratch" in _lib.last_error() and "4096 tokens" in _lib.last_error()
+        assert L.qmoe_layer_forward_static(h, FAKE, 95, FAKE, None, None) == QMOE_ERR_CAPACITY  # (94 run below)
         assert L.qmoe_layer_forward_static(h, FAKE, 0, FAKE, None, None) == QMOE_OK  # no-op
     finally:
         L.qmoe_layer_destroy(h)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("spec_name,sizes", [("QWEN35B", (40, 3)), ("QWEN35B", (10, 1)), ("CONFIG1", (32, 17)),
-                                             ("GEMMA4", (16, 5)), ("PADDED", (20, 3)), ("LISTS", (300, 130))])
+@pytest.mark.parametrize("spec_name,sizes", [("QWEN35B", (40, 3)), ("QWEN35B", (10, 1)), ("QWEN35B", (94, 80)),
+                                             ("CONFIG1", (32, 17)), ("GEMMA4", (16, 5)), ("PADDED", (20, 3)),
+                                             ("LISTS", (720, 130))])
 def test_static_forward_matches_workspace_forward(gpu, spec_name, sizes):
     import torch
 
@@ -40,8 +42,10 @@ def test_static_forward_matches_workspace_forward(gpu, spec_name, sizes):
     from qwenium_amd._lib import check, lib
 
     # PADDED: widths off the kernels' grid (the static scratch also holds the padded rows);
-    # LISTS: 300 tokens over 256 experts take the per-expert list launch and the MFMA GEMMs with
-    # their fixup list, then 130 tokens the merged top-k and the streaming GEMVs on the same scratch
+    # LISTS: 720 tokens over 256 experts take the batched router, the per-expert list launch and
+    # the f16 GEMMs with their fixup list, then 130 tokens the merged top-k and the int8 GEMMs, whose
+    # tile list lies where the fixup list was; (94, 80): the most that the scratch holds, and the most
+    # that it held when (gate, up) pairs had a buffer
     spec = (synthetic.LayerSpec(96, 8, 2, 32, True, synthetic.TYPE_Q4_0) if spec_name == "PADDED"
             else synthetic.LayerSpec(256, 256, 8, 64, True, synthetic.TYPE_Q4_0) if spec_name == "LISTS"
             else getattr(synthetic, spec_name))
