@@ -283,8 +283,7 @@ def run_leg(args, pool: LayerPool, workload: str, headline: bool) -> dict:
     ops_gu = 2.0 * R * 2 * F * H      # the GEMMs' multiply-adds x2 (quant x quant), gate + up
     ops_dn = 2.0 * R * H * F
     layer_ops = ops_gu + ops_dn
-    # the library's default switch to the f16-MFMA GEMMs: the rows that an expert averages (with copies)
-    mfma_path = T >= 128 and T * K >= (22 if spec.wtype == TYPE_Q4_0 else 28) * E
+    mfma_path = T >= layers[0].f16_min_tokens  # the f16-MFMA GEMMs (exact int8 ones below)
 
     log(f"warmup {warmup} steps")
     for i in range(warmup):

@@ -139,6 +139,10 @@ int qmoe_layer_create(const qmoe_tensor* w_router,
 int qmoe_layer_destroy(qmoe_layer* layer);
 /* n_embd of a created layer (ne[0] of w_router). */
 int qmoe_layer_n_embd(const qmoe_layer* layer);
+/* Token count from which the layer's forwards run the f16-MFMA expert GEMMs
+ * (f32 sums) in place of the exact ones; lower with prefill copies.  No
+ * counterpart in the reference: for profilers and tests. */
+int32_t qmoe_layer_f16_min_tokens(const qmoe_layer* layer);
 /* Reads the layer's expert tensors now (their data must be in place) and keeps
  * chunk-major copies of them for the prefill GEMMs (block pairs of one k chunk
  * of consecutive rows side by side), which then load a few cache lines per wave

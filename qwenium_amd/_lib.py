@@ -32,6 +32,7 @@ EXPORTED = (
     "qmoe_layer_create",
     "qmoe_layer_destroy",
     "qmoe_layer_n_embd",
+    "qmoe_layer_f16_min_tokens",
     "qmoe_layer_build_prefill_copies",
     "qmoe_workspace_create",
     "qmoe_workspace_destroy",
@@ -154,6 +155,8 @@ def lib() -> ctypes.CDLL:
     L.qmoe_layer_destroy.argtypes = [vp]
     L.qmoe_layer_n_embd.restype = ctypes.c_int
     L.qmoe_layer_n_embd.argtypes = [vp]
+    L.qmoe_layer_f16_min_tokens.restype = ctypes.c_int32
+    L.qmoe_layer_f16_min_tokens.argtypes = [vp]
     L.qmoe_layer_build_prefill_copies.restype = ctypes.c_int
     L.qmoe_layer_build_prefill_copies.argtypes = [vp]
     L.qmoe_workspace_create.restype = ctypes.c_int

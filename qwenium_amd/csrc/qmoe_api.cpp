@@ -486,6 +486,8 @@ int qmoe_layer_destroy(qmoe_layer* layer) {
 
 int qmoe_layer_n_embd(const qmoe_layer* layer) { return layer ? layer->Hu : 0; }
 
+int32_t qmoe_layer_f16_min_tokens(const qmoe_layer* layer) { return layer ? qmoe::mfma_from(layer->d) : 0; }
+
 int qmoe_workspace_create(const qmoe_layer* like, int32_t max_tokens, qmoe_workspace** out) {
     g_last_error.clear();
     if (!out) return fail(QMOE_ERR_NULL, "qmoe: out expected a non-null qmoe_workspace**, got null");

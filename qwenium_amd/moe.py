@@ -175,6 +175,11 @@ class MoELayer:
         self.n_embd = int(lib().qmoe_layer_n_embd(h))
         self._maybe_prefill_copies(prefill_copies, w_exp_gate)
 
+    @property
+    def f16_min_tokens(self) -> int:
+        """Token count from which forwards run the f16-MFMA expert GEMMs (the exact ones below)."""
+        return int(lib().qmoe_layer_f16_min_tokens(self._handle))
+
     def _maybe_prefill_copies(self, wanted: bool, probe: GGMLTensor) -> None:
         # the copies read the weights now: only for device-resident tensors, and not
         # when QMOE_PREFILL_REPACK=0 (the prefill GEMMs then read the GGUF rows)

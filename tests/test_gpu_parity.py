@@ -3,12 +3,12 @@ same seeded inputs.
 
 Bar: top-k expert ids, per-expert offsets and row lists bit-exact (ties to the
 lowest expert id); layer outputs within max-abs 2e-3 x output RMS.  Below the
-MFMA threshold the kernels accumulate quantized block dots exactly (f64) and use the
+f16 threshold the kernels accumulate quantized block dots exactly (f64) and use the
 same deterministic exp, so outputs are in practice bit-identical; that is
 asserted separately as a fraction so a rare router rounding flip does not hide
-behind it.  From max(128, 5.5 n_experts / top_k) tokens (176 at the 35B-A3B shape) or when
-forced, the grouped GEMMs run f16 MFMAs:
-the block dots are exact, their scaled sum is accumulated in f32, and every h
+behind it.  From MoELayer.f16_min_tokens on (22 rows per expert in Q4_0 and 28 in Q8_0
+with prefill copies, 36 and 56 without; 128 tokens at least) or when forced, the grouped
+GEMMs run f16 MFMAs: the block dots are exact, their scaled sum is accumulated in f32, and every h
 value whose Q8_0 rounding that error could change is recomputed exactly, so the
 h quants match the oracle's; outputs differ by f32 rounding of the sums (about
 1e-6 x RMS), held to MFMA_TOL, a hundred times tighter than the bar.
@@ -40,9 +40,9 @@ def host_layer(spec: LayerSpec, tensors: dict) -> po.Layer:
     return po.Layer(spec.n_embd, spec.n_experts, spec.top_k, spec.ffn_dim, spec.shared, spec.wtype, host)
 
 
-def run_pair(spec: LayerSpec, T: int, seed: int, batch: int = 0, x=None):
+def run_pair(spec: LayerSpec, T: int, seed: int, batch: int = 0, x=None, copies: bool = True):
     tensors = synthetic.make_layer_tensors(spec, seed)
-    layer = synthetic.make_layer(spec, seed, tensors=tensors)
+    layer = synthetic.make_layer(spec, seed, tensors=tensors, prefill_copies=copies)
     if x is None:
         x = synthetic.make_x(spec, T, seed, batch)
     y, dbg = layer.forward(x, debug=True)
@@ -135,14 +135,21 @@ def test_decode_35b_token_counts(gpu, spec, T):
     assert_parity(y, got, y_ref, d_ref, spec)
 
 
-@pytest.mark.parametrize("T", [160, 175, 176])
-def test_35b_around_mfma_threshold(gpu, T):
-    """The 35B shape switches to the f16-MFMA GEMMs where an expert averages 5.5 rows
-    (176 tokens): 160 and 175 tokens stream (outputs bit-identical to the oracle), 176 runs
-    the MFMA GEMMs (h quants exact, outputs within MFMA_TOL); routing bit-exact on all."""
-    spec = synthetic.QWEN35B
-    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=500 + T)
-    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= 176, min_identical=1.0)
+@pytest.mark.parametrize("wtype,copies,T,f16_from", [
+    (TYPE_Q4_0, True, 160, 704), (TYPE_Q4_0, True, 176, 704), (TYPE_Q4_0, True, 703, 704), (TYPE_Q4_0, True, 704, 704),
+    (TYPE_Q4_0, False, 1151, 1152), (TYPE_Q4_0, False, 1152, 1152),
+    (TYPE_Q8_0, True, 895, 896), (TYPE_Q8_0, True, 896, 896),
+    (TYPE_Q8_0, False, 1791, 1792), (TYPE_Q8_0, False, 1792, 1792)])
+def test_35b_around_mfma_threshold(gpu, wtype, copies, T, f16_from):
+    """The 35B shape switches to the f16-MFMA GEMMs where an expert averages 22 rows (Q4_0 with
+    prefill copies), 36 (without), 28 or 56 (Q8_0): one token below, the exact int8 GEMMs give
+    the oracle's bits; at the switch the f16 GEMMs list h blocks for their fixup, h quants are
+    exact and outputs within MFMA_TOL; routing bit-exact on all."""
+    spec = synthetic.QWEN35B if wtype == TYPE_Q4_0 else synthetic.QWEN35B_Q8
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=500 + T, copies=copies)
+    assert layer.f16_min_tokens == f16_from
+    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= f16_from, min_identical=1.0)
+    assert (got["h_fixed"][0] > 0) == (T >= f16_from)
 
 
 @pytest.mark.parametrize("spec,T", [(LayerSpec(4096, 64, 4, 256, True, TYPE_Q8_0), 7),
@@ -176,11 +183,11 @@ def test_padded_widths(gpu, spec, T):
     """n_embd and ffn_dim that Q4_0/Q8_0 rows allow (multiples of 32) but the kernels'
     grid does not (multiples of 256 and 64): the layer runs on zero-padded weight copies
     and zero-padded rows, and routing and outputs match the oracle at the caller's widths
-    as on every other path (decode, streaming, MFMA with the grouped router (300 tokens)
-    and with the batched router (1100 tokens: from 1024 at these widths))."""
+    as on every other path (decode, the int8 GEMMs (17 and 150 tokens), the f16 GEMMs below the
+    batched router (300 tokens) and with it (1100))."""
     y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=400 + T)
     assert layer.n_embd == spec.n_embd and y.shape == (T, spec.n_embd)
-    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= 128)
+    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= layer.f16_min_tokens)
 
 
 @pytest.mark.parametrize("spec,T", [(LayerSpec(256, 256, 16, 64, True, TYPE_Q4_0), 300),
@@ -190,9 +197,10 @@ def test_expert_lists_wide_top_k(gpu, spec, T):
     """The per-expert lists built from the top-k blocks' token masks (top-k blocks x experts
     above 4096) at top_k 16, 17 and 24: each listed token's slot comes from the four-bit
     fields that the top-k writes up to top_k 16 and from a search of the token's selection
-    above it; grouped router (300 tokens) and batched router (1100 tokens)."""
-    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=450 + spec.top_k)
-    assert_parity(y, got, y_ref, d_ref, spec, mfma=True)
+    above it; f64-MFMA router and int8 GEMMs (300 tokens), batched router and f16 GEMMs (1100)."""
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=450 + spec.top_k)
+    assert (T >= layer.f16_min_tokens) == (T == 1100)
+    assert_parity(y, got, y_ref, d_ref, spec, mfma=T == 1100)
 
 
 @pytest.mark.parametrize("T", [1, 2, 15, 16, 17, 33, 64])
@@ -355,13 +363,15 @@ def test_graph_replay_matches_eager(gpu):
         torch.cuda.synchronize()
 
 
-def test_graph_replay_prefill_matches_eager(gpu):
-    """Prefill forwards (batched router, f16-MFMA GEMMs, fixups) captured in a
-    HIP graph: every replay equals the eager result bit for bit."""
+@pytest.mark.parametrize("T", [40, 512, 720])
+def test_graph_replay_prefill_matches_eager(gpu, T):
+    """Forwards past decode captured in a HIP graph: every replay equals the eager result bit
+    for bit.  40 and 512 tokens: f64-MFMA router, int8 GEMMs (the merged top-k, whose last
+    workgroup builds the lists, and the list launch); 720: batched router, f16-MFMA GEMMs, fixups."""
     from qwenium_amd import Workspace
     spec = synthetic.QWEN35B
-    T = 512
     layers = [synthetic.make_layer(spec, 70 + i) for i in range(2)]
+    assert (T >= layers[0].f16_min_tokens) == (T == 720)
     xs = [synthetic.make_x(spec, T, 70, batch=b) for b in range(2)]
     ws = Workspace(layers[0], T)
     eager = [layers[i].forward(xs[i], workspace=ws).clone() for i in range(2)]
@@ -401,7 +411,8 @@ def test_mfma_config1_forced(gpu, monkeypatch):
     assert_parity(y, got, y_ref, d_ref, spec, mfma=True)
 
 
-def test_mfma_35b_q4_0_t256(gpu):
+def test_mfma_35b_q4_0_t256(gpu, monkeypatch):
+    monkeypatch.setenv("QMOE_MFMA_MIN_TOKENS", "256")
     spec = synthetic.QWEN35B
     y, got, y_ref, d_ref, *_ = run_pair(spec, 256, seed=9)
     assert_parity(y, got, y_ref, d_ref, spec, mfma=True)
@@ -424,8 +435,8 @@ def test_batched_router_forced_small_layer(gpu, monkeypatch, T):
     experts (E=16 < one 64-expert tile)."""
     monkeypatch.setenv("QMOE_BIG_ROUTER_MIN_TOKENS", "1")
     spec = LayerSpec(256, 16, 4, 128, True, TYPE_Q4_0)
-    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=300 + T)
-    assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0, mfma=T >= 128)
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=300 + T)
+    assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0, mfma=T >= layer.f16_min_tokens)
     check_router_bound(got, d_ref["logits"])
 
 
@@ -435,8 +446,8 @@ def test_router_threshold_35b(gpu, T):
     from 720, with debug buffers as without them: both give the oracle's routing, and only
     the batched one writes approximate logits and bounds."""
     spec = synthetic.QWEN35B
-    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=31)
-    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= 704)  # (22 rows per expert: the f16 GEMMs)
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=31)
+    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= layer.f16_min_tokens)
     if T >= 720:
         assert check_router_bound(got, d_ref["logits"]) < 0.5
     else:
@@ -662,7 +673,7 @@ def test_fused_decode_routing_repeated(gpu, n_experts, T):
 
 def _random_cases(n=32, seed=2024):
     """Seeded layer shapes and token counts across every path (decode, grouped
-    router + streaming, MFMA GEMMs, batched router), padded widths and both
+    router + int8 GEMMs, f16 GEMMs, batched router), padded widths and both
     weight types; fixed at import, so the parametrization is stable."""
     rng = np.random.default_rng(seed)
     cases = []
@@ -679,18 +690,12 @@ def _random_cases(n=32, seed=2024):
     return cases
 
 
-def _mfma_min_tokens(spec: LayerSpec) -> int:
-    t = (11 * spec.n_experts + 2 * spec.top_k - 1) // (2 * spec.top_k)
-    return max(128, min(4096, (t + 15) // 16 * 16))
-
-
 @pytest.mark.parametrize("spec,T", _random_cases())
 def test_random_shapes(gpu, spec, T):
     """Seeded random shapes against the oracle: routing bit-exact; outputs bit-identical
-    below the MFMA threshold (max(128, 5.5 n_experts / top_k) tokens), within MFMA_TOL
-    with exact h quants above it."""
-    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=700 + T)
-    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= _mfma_min_tokens(spec), min_identical=1.0)
+    below the f16 threshold, within MFMA_TOL with exact h quants from it on."""
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=700 + T)
+    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= layer.f16_min_tokens, min_identical=1.0)
 
 
 def _random_prefill_cases(n=48, seed=12):
@@ -717,9 +722,9 @@ def _random_prefill_cases(n=48, seed=12):
 @pytest.mark.parametrize("spec,T", _random_prefill_cases())
 def test_random_prefill_shapes(gpu, spec, T):
     """Seeded prefill-size shapes against the oracle: routing and lists bit-exact, h quants
-    exact and outputs within MFMA_TOL on the MFMA path (bit-identical below it)."""
-    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=800 + T)
-    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= _mfma_min_tokens(spec), min_identical=1.0)
+    exact and outputs within MFMA_TOL on the f16 path (bit-identical below it)."""
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=800 + T)
+    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= layer.f16_min_tokens, min_identical=1.0)
 
 
 def _chain_cases(n=12, seed=77):
@@ -764,12 +769,13 @@ def test_forward_norm_chain_random(gpu, spec, T):
 
 @pytest.mark.parametrize("T", [300, 720, 800])
 def test_1024_experts_prefill(gpu, monkeypatch, T):
-    """1024 experts (the most a layer takes): the grouped router with the streaming GEMVs
-    (300 tokens), the f16-MFMA GEMMs (from 5.5 * 1024 / 8 = 704 tokens) with the grouped
-    router (720) and with the batched router (800 tokens; its threshold held at 784 here,
-    above the shape's own 320, so that both routers meet the MFMA GEMMs), sixteen 64-expert
-    router tiles and the per-expert lists."""
+    """1024 experts (the most a layer takes): the f64-MFMA router with the int8 GEMMs (300
+    tokens), the f16-MFMA GEMMs (held at 704 tokens here, below the shape's own 2816) with
+    the f64-MFMA router (720) and with the batched router (800 tokens; its threshold held at
+    784, so that both routers meet the f16 GEMMs), sixteen 64-expert router tiles and the
+    per-expert lists."""
     monkeypatch.setenv("QMOE_BIG_ROUTER_MIN_TOKENS", "784")
+    monkeypatch.setenv("QMOE_MFMA_MIN_TOKENS", "704")
     spec = LayerSpec(256, 1024, 8, 64, True, TYPE_Q4_0)
     y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=600 + T)
     assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= 704, min_identical=1.0)
@@ -818,8 +824,7 @@ def test_forward_norm_chain(gpu, which, T):
 def test_forward_norm_matches_unfused(gpu, which, T):
     """y = x + MoE(RMSNorm(x) * w) in one call (the decode routing normalizes while it
     stages x, the batched router's preparation and refinement normalize from its
-    threshold on (224 tokens at the 35B-A3B shape), other sizes normalize into the
-    workspace) gives the bits of rms_norm
+    threshold on (720 tokens), other sizes normalize into the workspace) gives the bits of rms_norm
     followed by forward(residual=x)."""
     from qwenium_amd import Workspace, rms_norm
 
@@ -1002,5 +1007,5 @@ def test_row_pair_router_groups(gpu, hidden, experts, T):
     most blocks before the f64-MFMA tiles take over (33 x 7 against 33 x 8): logits within one
     ulp of the oracle's, routing and outputs equal."""
     spec = LayerSpec(hidden, experts, min(2, experts), 64, True, TYPE_Q8_0)
-    y, got, y_ref, d_ref, *_ = run_pair(spec, T, seed=600 + T)
-    assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0, mfma=T * 2 >= 28 * experts and T >= 128)
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=600 + T)
+    assert_parity(y, got, y_ref, d_ref, spec, min_identical=1.0, mfma=T >= layer.f16_min_tokens)
