@@ -474,11 +474,13 @@ bool down_combine_tok_fits(const LayerDesc& L) {
 // Whether reading each token's experts' down rows for it alone (the token-per-
 // workgroup kernel, ~8.7 TB/s out of the caches) beats reading each expert's once
 // (the grouped GEMM at ~4.5 TB/s and its combine's ~8 us).  Layer us, token /
-// grouped: 35B-A3B Q4_0 93.4 / 99.4 at 32 tokens, 123.0 / 123.3 at 64, 147.7 /
-// 140.8 at 96; Q8_0 196.7 / 194.6 at 64; Gemma 4 109.7 / 116.6 at 24, 142.6 /
-// 135.8 at 48; hidden 4096, 32 experts, top-4 78.4 / 77.4 at 17, 114.0 / 88.5 at
-// 48.  From four rows per expert and 40 tokens always grouped, small layers too
-// (hidden 1024, 16 experts, top-2 35.7 / 36.6 at 32, 40.9 / 38.1 at 48).
+// grouped: 35B-A3B Q4_0 87.7 / 95.5 at 32 tokens, 114.6 / 115.5 at 64, 131.1 /
+// 125.6 at 96; Q8_0 157.6 / 157.1 at 48, 180.1 / 171.7 at 64; Gemma 4 121.8 / 122.9
+// at 32, 131.3 / 127.8 at 40; hidden 4096, 32 experts, top-4 77.7 / 76.8 at 17,
+// 84.9 / 77.1 at 24.  The model leaves small layers to the token kernel too long
+// (8.7 TB/s is not reached there): from four rows per expert and 40 tokens always
+// grouped (hidden 1024, 16 experts, top-2, Q8_0 31.3 / 29.0 at 32, 36.7 / 30.2 at 48;
+// Q4_0 25.7 / 26.3 at 32, 28.4 / 27.5 at 48; hidden 512 23.4 / 25.9 at 40).
 static bool down_per_token(const LayerDesc& L, int T) {
     if (T >= 40 && (int64_t)T * L.K >= 4 * (int64_t)L.E) return false;
     const int bb = L.dn_type == kTypeQ4_0 ? BlockTraits<kTypeQ4_0>::kBytes : BlockTraits<kTypeQ8_0>::kBytes;

@@ -475,12 +475,19 @@ static I8Args base_i8_args(const LayerDesc& L, const Workspace& ws) {
     return a;
 }
 
-// 16 rows per workgroup (three workgroups per CU) up to 14 rows per expert, 32 (two)
-// beyond, where 16 would read the weights of most experts twice.  Layer us, 16 / 32:
-// 35B-A3B Q4_0 179 / 187 at 9 rows, 208 / 211 at 14, 270 / 256 at 22; Q8_0 265 / 263
-// at 14, 353 / 305 at 22; Gemma 4 202 / 200 at 12, 252 / 240 at 19.
+// 16 rows per workgroup (three workgroups per CU) at few rows per expert, 32 beyond, where 16
+// would read the weights of most experts twice: from 14 rows in Q8_0 (two workgroups per CU), from
+// 8 in Q4_0, whose 32-row gate/up fits three as well, except where the shared expert's full tiles,
+// twice as long then, outlast a small grid (fewer than four workgroups per CU).  Layer us, 16 / 32:
+// 35B-A3B Q4_0 139.8 / 141.0 at 5 rows, 162.6 / 154.4 at 8, 198.0 / 185.6 at 14; Gemma 4 135.9 /
+// 139.3 at 4, 161.8 / 156.4 at 8; 128 experts of ffn 1536, hidden 4096 318.3 / 328.5 at 6, 345.7 /
+// 345.8 at 8; 32 of ffn 512, hidden 2048 45.9 / 42.4 at 8, 53.1 / 48.1 at 11, with a shared expert
+// 54.2 / 56.4 and 56.0 / 59.4; Q8_0 218.9 / 231.6 at 9, 254.8 / 249.2 at 14, Gemma 4 208.7 / 214.5
+// at 10, 226.8 / 223.8 at 12.5.
 int i8_tile_rows(const LayerDesc& L, int T) {
-    return (int64_t)T * L.K > 14 * (int64_t)L.E ? 32 : 16;
+    const bool full_grid = (int64_t)L.E * (L.F / 64) >= 4 * (int64_t)L.n_cu;
+    const int from = L.gu_type == kTypeQ4_0 && (!L.S || full_grid) ? 8 : 14;
+    return (int64_t)T * L.K > from * (int64_t)L.E ? 32 : 16;
 }
 
 template <int WT, bool GATEUP, int ROWS, bool TAIL, int CW, int KS>

@@ -378,11 +378,18 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
     // token count from which the grouped f16-MFMA GEMMs (f32 sums, 128-row tiles)
     // replace the exact int8 ones: by the rows that an expert averages (T * top_k /
     // n_experts), 36 (Q4_0) or 56 (Q8_0) over the GGUF rows, 22 or 28 with the
-    // chunk-major copies.  Layer us, int8 / f16: 35B-A3B Q4_0 332 / 358 at 31 rows,
-    // 388 / 385 at 37, with copies 245 / 262 at 19 and 332 / 293 at 31; Q8_0 504 /
-    // 537 at 47, with copies 326 / 339 at 25 and 385 / 360 at 31; Gemma 4 Q4_0 293 /
-    // 328 at 28, 360 / 346 at 37, with copies 219 / 230 at 16 and 255 / 243 at 22;
-    // Q8_0 526 / 549 at 62, 613 / 582 at 75, with copies 321 / 325 at 28.
+    // chunk-major copies.  Layer us, int8 / f16: 35B-A3B Q4_0 359 / 380 at 36 rows,
+    // 385 / 394 at 41, with copies 219 / 259 at 19, 239 / 258 at 22 and 307 / 292 at 31;
+    // Q8_0 495 / 533 at 44, 573 / 561 at 56, with copies 297 / 332 at 22, 347 / 350 at
+    // 28 and 426 / 383 at 34; Gemma 4 Q4_0 253 / 311 at 28, 349 / 345 at 44, with
+    // copies 188 / 197 at 16 and 215 / 206 at 22; Q8_0 478 / 500 at 56, 575 / 539 at
+    // 69, with copies 267 / 282 at 25 and 345 / 309 at 32; skewed routing (half of the
+    // rows on 8 of 256 experts) Q4_0 340 / 386 at 36, with copies 246 / 256 at 22, Q8_0
+    // 564 / 589 at 56, with copies 354 / 339 at 28; hidden 4096, 32 experts, Q4_0 154 /
+    // 172 at 30, 192 / 187 at 35, with copies 123 / 131 at 22, 147 / 137 at 25, Q8_0
+    // with copies 153 / 159 at 22, 184 / 164 at 25 (a second round of workgroups: the
+    // line is late there).  Few workgroups keep the int8 GEMMs ahead longer than this
+    // says: hidden 1024, 16 experts, Q8_0 55 / 72 at 56 rows, 82 / 85 at 125.
     {
         const bool q4 = d.gu_type == QMOE_TYPE_Q4_0;
         auto from = [&](int rows) {

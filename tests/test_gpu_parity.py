@@ -903,8 +903,9 @@ def test_python_checks_on_device_operands(gpu):
     # all rows on one expert: 32-row tiles whose last group of four rows is full or holds one row
     (1, 1, 17), (1, 1, 20), (1, 1, 21), (1, 1, 24), (1, 1, 25), (1, 1, 28), (1, 1, 29), (1, 1, 31), (1, 1, 32),
     (1, 1, 33), (1, 1, 129),
-    (16, 2, 17), (16, 2, 40), (16, 2, 112), (16, 2, 113),  # 1 to ~20 rows, both tile heights
+    (16, 2, 17), (16, 2, 40), (16, 2, 112), (16, 2, 113),  # 1 to ~20 rows, both tile heights (from 14 rows)
     (64, 4, 40), (64, 4, 300),                             # grids past the CUs at ffn 576 and 704
+    (96, 6, 128), (96, 6, 129),                            # at ffn 704 32-row tiles from 8 rows in Q4_0
 ])
 def test_i8_experts_tile_edges(gpu, monkeypatch, wtype, hidden, ffn, experts, top_k, T):
     """Tiles of 16 and 32 rows at both ends of every group of four, reduction lengths that end
