@@ -99,9 +99,9 @@ typedef struct qmoe_debug {
     /* [T*top_k + S*T][n_embd] the unweighted expert rows, the reference's
      * moe_exp_down (moe.cpp:127-128) and moe_shared_out (:165), same row
      * order as h.  Written only where the forward materializes them (the
-     * f16-MFMA path and the streaming path without the fused combine); at
-     * decode sizes the combine consumes them in registers and this buffer is
-     * left as it was. */
+     * f16-MFMA and int8-MFMA down projections); where the down projection runs
+     * per token with the combine in it (decode sizes and somewhat above), the
+     * combine consumes them in registers and this buffer is left as it was. */
     float*   exp_down;
 } qmoe_debug;
 

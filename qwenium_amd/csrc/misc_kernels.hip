@@ -169,8 +169,8 @@ hipError_t launch_fill_i32(int32_t* dst, int n, int32_t v, hipStream_t stream) {
 // Debug copies of per-row intermediates in assignment order.  Workspace row p
 // holds routed assignment rows[p] for p < A (rows grouped by expert) and the
 // shared expert's row of token p - A after them; output row = rows[p] or p.
-// h: from the int8 quants + {d, sum} records of the decode and streaming paths
-// (qs8, ds8) or the f16 quants + fp16 scale bits of the MFMA path (q16, d16);
+// h: from the int8 quants + {d, sum} records of the decode and int8 GEMM paths
+// (qs8, ds8) or the f16 quants + fp16 scale bits of the f16 path (q16, d16);
 // the first fo of each f-wide row (fo: the caller's ffn width).
 __global__ __launch_bounds__(256) void k_debug_h(const int32_t* rows, int A, int R, int f, int fo, const int8_t* qs8,
                                                  const float2* ds8, const _Float16* q16, const uint16_t* d16,

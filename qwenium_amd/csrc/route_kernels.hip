@@ -16,8 +16,8 @@ namespace qmoe {
 // ---------------------------------------------------------------------------
 // R1: exact router logits of every token, for the debug copy when the batched
 // router runs (its own logits are approximate); the forward paths compute
-// theirs in k_route_decode (up to 16 tokens) and k_router_group (up to the batched
-// router's threshold) or refine the batched router's candidates in k_topk
+// theirs in k_route_decode (up to 16 tokens, and beyond while its blocks fill the CUs
+// once at most) and k_router_group (up to the batched router's threshold) or refine the batched router's candidates in k_topk
 // ---------------------------------------------------------------------------
 struct RouterArgs {
     const float* x;         // [T][H] router input
@@ -1567,7 +1567,8 @@ __global__ __launch_bounds__(1024) void k_route_decode(TopkArgs a, float* logits
     }
 }
 
-// The router from 17 tokens to the batched router's threshold: one workgroup per 16
+// The router from 17 tokens to the batched router's threshold (router_in_row_pairs says
+// where k_route_decode's groups run instead): one workgroup per 16
 // tokens x 16 experts (the shared gate the last column), logits from
 // v_mfma_f64_16x16x4_f64 on the f32 operands widened, so each product is exact and
 // the sum is f64 as everywhere.  A matrix instruction does 16 vector FMAs' work in
@@ -1637,7 +1638,7 @@ __global__ __launch_bounds__(1024) void k_router_group(TopkArgs a, float* logits
 
 // Decode routing on the router launch's logits (complete and visible at the
 // launch boundary): workgroup 0 runs the top-k, softmax, counts, scan and the
-// row and slot tables; the other workgroups meanwhile compute the shared
+// row tables and the decode slot list; the other workgroups meanwhile compute the shared
 // expert's h (SWT: its weight type) or, without one, x's Q8_0 (one wave per token).
 template <int SWT, int SLPR>
 __global__ __launch_bounds__(1024) void k_route_decode_tables(TopkArgs a, int8_t* xq_qs, float2* xq_ds, SharedGuArgs sg) {
