@@ -360,11 +360,10 @@ __global__ __launch_bounds__(64 * CW * KS, i8_waves_per_simd(WT, GATEUP, ROWS, K
                 if (live) put(c);  // (the wave's own slab)
                 if (stage) __syncthreads();
                 else wave_lds_order();
-                if (c + KS < nchunk) {
-                    fetch(cg, c + KS);
-                    fetch_a(c + KS);
-                } else if (cg + 1 < ncg) {
-                    fetch(cg + 1, 0);
+                const bool last = c + KS >= nchunk;
+                if (!last || cg + 1 < ncg) {  // (one place that fetches: two are twice the code)
+                    fetch(last ? cg + 1 : cg, last ? 0 : c + KS);
+                    if (nstep > 1) fetch_a(last ? 0 : c + KS);
                 }
                 const int np = !live ? 0 : TAIL ? min(kPairs, npairs - kPairs * c) : kPairs;
 #pragma unroll 1
