@@ -21,9 +21,10 @@
 // exist; two waves with half of a Q8_0 block of h each instead of one with all of
 // it keep the workgroups short (the last round of them costs a workgroup's time).
 // Measured, 35B-A3B shape, us: gate/up at 211 tokens Q4_0 217 (f16 path, GGUF rows)
-// -> 82 (3.7 TB/s), down 84 -> 44; gate/up at 64 tokens 85 (streaming GEMV and the
-// Q8_0 of h) -> 63 (4.2 TB/s); gate/up at 512 tokens Q8_0 207 + 12 of fixups (f16
-// path with copies) -> 154, down 97 -> 78.
+// -> 79 (353 MB fetched, 4.5 TB/s; VALU issue is 49% of its cycles), down 84 -> 43;
+// gate/up at 64 tokens 85 (streaming GEMV and the Q8_0 of h) -> 59; at 1000 tokens 161
+// (2.9 TB/s, VALU issue 65%), down 84; at 512 tokens Q8_0 207 + 12 of fixups (f16 path
+// with copies) -> 154, down 97 -> 78.
 #include "qmoe_device.h"
 #include "qmoe_internal.h"
 
@@ -53,7 +54,8 @@ constexpr int i8_waves_per_simd(int wt, bool gateup, int rows, int ks) {
 
 // a workgroup of at most ROWS (16 or 32) rows of one expert, chunks of P pairs: a chunk's
 // activation quants [pair][lane group][slot][16 bytes] and block scales [block][slot], padded
-// so that neither the staging writes nor the operand reads meet in a bank
+// against bank conflicts (a third of the gate/up's LDS cycles still conflict, with its LDS
+// instructions 3 to 4% of the wave-cycles)
 template <int ROWS> constexpr int kI8APair = 4 * ROWS * 16 + 16;
 template <int ROWS> constexpr int kI8DBlock = ROWS + 4;
 template <int P, int ROWS> constexpr int kI8ABytes = P * kI8APair<ROWS>;
@@ -61,7 +63,7 @@ template <int P, int ROWS> constexpr int kI8DBytes = 2 * P * kI8DBlock<ROWS> * 4
 
 template <int WT> constexpr int kI8PairBytes = 2 * BlockTraits<WT>::kBytes;
 template <int WT, int P> constexpr int kI8RowBytes = P * kI8PairBytes<WT>;  // of a chunk
-// LDS row stride: 36, 76 or 68 dwords (columns 16 apart in four banks each way)
+// LDS row stride: 36, 76 or 68 dwords
 template <int WT, int P> constexpr int kI8Ld = kI8RowBytes<WT, P> + (kI8RowBytes<WT, P> == 288 ? 16 : 0);
 template <int WT, int P> constexpr int kI8WBytes = 32 * kI8Ld<WT, P>;       // a wave's weight slab: 32 columns
 template <int WT, int P, int ROWS, int CW>  // CW waves' weight slabs and their chunk's activations
