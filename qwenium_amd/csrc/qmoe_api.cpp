@@ -400,12 +400,20 @@ int qmoe_layer_create(const qmoe_tensor* w_router, const qmoe_tensor* w_exp_gate
         d.mfma_min_tokens_pk = from(q4 ? 22 : 28);
     }
     // token count from which routing runs the batched bf16-MFMA router with its exact
-    // refinement in place of the f64-MFMA one: layer us, f64 / batched, 35B-A3B shape 219
-    // / 227 at 600 tokens, 284 / 283 at 800, 310 / 299 at 1000; Gemma 4 325 / 333 at 800,
-    // 432 / 426 at 1200; 512 experts of 1024 columns 172 / 176 at 800, 188 / 184 at 1000;
-    // 64 experts of 1536 165 / 169 at 600, 206 / 201 at 1000 (the crossings lie from 700
-    // tokens, with the RMSNorm folded into the batched router's preparation, to 1200)
-    d.big_router_min_tokens = 720;
+    // refinement in place of the exact ones: 720, fewer for routers of more than 655360
+    // weights, whose f64 products grow faster than the refinement's rows.  Layer us, exact /
+    // batched: 35B-A3B shape 219 / 227 at 600 tokens, 284 / 283 at 800, 310 / 299 at 1000;
+    // Gemma 4 325 / 333 at 800, 432 / 426 at 1200; 64 experts of 1536 columns 165 / 169 at
+    // 600, 206 / 201 at 1000; 16 of 4096 level past 1000.  1024 experts of 4096 columns (400)
+    // +4% at 288 tokens, -2% at 336, -12% at 576; 512 of 4096 (496) +2% at 336, -4% at 480,
+    // -8% at 704; 1024 of 2048 (496) +2% at 432, -8% at 480; 768 of 2048 (544) +3% at 480,
+    // level at 528, -6% at 704; 1024 of 1024 (624) +3% at 528, +1% at 576, -3% at 640; 512 of
+    // 2048 (624) +1% at 576, -3% at 640; with the RMSNorm in the call, which the batched
+    // router's preparation folds in, up to 4% more.
+    {
+        const double t = 720.0 * std::min(1.0, std::cbrt(655360.0 / ((double)d.E * (double)d.H)));
+        d.big_router_min_tokens = (int)(std::ceil(t / 16.0) * 16.0);
+    }
     if (const char* env = std::getenv("QMOE_MFMA_MIN_TOKENS")) {
         const long v = std::strtol(env, nullptr, 10);
         if (v >= 1) d.mfma_min_tokens = d.mfma_min_tokens_pk = (int)std::min<long>(v, 1 << 30);

@@ -454,6 +454,20 @@ def test_router_threshold_35b(gpu, T):
         assert not np.isfinite(got["router_approx"]).any(), "the batched router ran below its threshold"
 
 
+@pytest.mark.parametrize("hidden,experts,T,batched", [(1024, 1024, 623, False), (1024, 1024, 624, True),
+                                                      (4096, 1024, 399, False), (4096, 1024, 400, True)])
+def test_router_threshold_large(gpu, hidden, experts, T, batched):
+    """Routers of more than 655360 weights: the batched one runs from 720 tokens times the cube
+    root of 655360 / weights, in steps of 16; the oracle's routing on both sides."""
+    spec = LayerSpec(hidden, experts, 2, 64, False, TYPE_Q4_0)
+    y, got, y_ref, d_ref, layer, *_ = run_pair(spec, T, seed=33)
+    assert_parity(y, got, y_ref, d_ref, spec, mfma=T >= layer.f16_min_tokens)
+    if batched:
+        check_router_bound(got, d_ref["logits"])
+    else:
+        assert not np.isfinite(got["router_approx"]).any()
+
+
 @pytest.mark.parametrize("dup", ["pairs", "all"])
 def test_batched_router_ties(gpu, monkeypatch, dup):
     """Exactly tied logits through the refinement: duplicated router rows ("pairs"), or
