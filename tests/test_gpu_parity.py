@@ -363,13 +363,15 @@ def test_graph_replay_matches_eager(gpu):
         torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("T", [40, 512, 720])
-def test_graph_replay_prefill_matches_eager(gpu, T):
+@pytest.mark.parametrize("spec,T", [(synthetic.QWEN35B, 40), (synthetic.QWEN35B, 512), (synthetic.QWEN35B, 720),
+                                    (LayerSpec(4096, 16, 2, 128, True, TYPE_Q8_0), 17)])
+def test_graph_replay_prefill_matches_eager(gpu, spec, T):
     """Forwards past decode captured in a HIP graph: every replay equals the eager result bit
     for bit.  40 and 512 tokens: f64-MFMA router, int8 GEMMs (the merged top-k, whose last
-    workgroup builds the lists, and the list launch); 720: batched router, f16-MFMA GEMMs, fixups."""
+    workgroup builds the lists, and the list launch); 720: batched router, f16-MFMA GEMMs,
+    fixups; the small layer: the router's row pairs, gate/up workgroups split in four parts
+    (above 64 KiB of LDS)."""
     from qwenium_amd import Workspace
-    spec = synthetic.QWEN35B
     layers = [synthetic.make_layer(spec, 70 + i) for i in range(2)]
     assert (T >= layers[0].f16_min_tokens) == (T == 720)
     xs = [synthetic.make_x(spec, T, 70, batch=b) for b in range(2)]
